@@ -26,15 +26,13 @@
 #include <mutex>
 #include <type_traits>
 
-#include "nvjsel_device.h"
-#include "nvjsel_host.h"
+#include "lm_head_common.h"
 
 // Launch shapes (chosen by measurement on MI355X).
 static constexpr int kLmWaves = 8;  // waves per block
 static constexpr int kLmMt1 = 4;  // 16-row vocab tiles per wave when B <= 16
 static constexpr int kLmMtn = 2;  // ... when B > 16
 static constexpr int kLmKu = 4;  // 32-wide k-steps per prefetch chunk
-static constexpr int kLmNt = 1;  // non-temporal (streaming) loads of W
 static constexpr int kLmDepth = 3;  // k-chunks of W in flight per wave
 static constexpr int kLmBpc = 0;  // blocks per CU (0 = as many as occupancy allows)
 
@@ -46,228 +44,6 @@ static constexpr int kGemvR = 4;  // rows per wave step of the streaming GEMV
 static constexpr bool kGemvDot = true;  // bf16 hidden without prologue: v_dot2c_f32_bf16
 
 namespace nvjsel {
-
-template <typename T>
-__device__ __forceinline__ T stream_load(const T* p) {
-  if constexpr (kLmNt) return __builtin_nontemporal_load(p);
-  else return *p;
-}
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-// GREEDY: argmax id per row; SAMPLE: Gumbel-max id per row; LOGITS: the
-// (REDUCE_CAST-rounded) logits themselves, written to out_logits.
-enum { MODE_GREEDY = 0, MODE_SAMPLE = 1, MODE_LOGITS = 2 };
-
-struct LmArgs {
-  const void* W;
-  const void* hidden;
-  int hidden_dtype;    // element type of `hidden` as stored
-  // final RMSNorm prologue (prenorm != 0): the kernel multiplies against
-  // act(in(rms_norm(hidden) * (1 + norm_w))) instead of `hidden`
-  int prenorm;
-  const void* norm_w;
-  int norm_dtype;
-  float eps;
-  int act_dtype;
-  int weight_dtype;
-  int layout;
-  int B;  // rows handled by this launch
-  int H;
-  int V;
-  int reduce_cast;
-  const float* temperature;  // MODE_SAMPLE, offset to this launch's first row
-  const uint32_t* keys;      // MODE_SAMPLE, [B,2]
-  unsigned long long* row_keys;
-  unsigned int* counter;
-  int32_t* out_ids;
-  float* out_best;
-  void* out_logits;      // MODE_LOGITS: [B, out_stride] of out_dtype, offset to this launch's first row
-  int out_dtype;         // DT_F32, DT_BF16 or DT_F16
-  long long out_stride;  // elements between output rows
-};
-
-// MODE_LOGITS store of logit (b, v): f32 as is, bf16 / f16 rounded to nearest even.
-__device__ __forceinline__ void store_logit(const LmArgs& a, int b, int v, float val) {
-  const size_t i = (size_t)b * (size_t)a.out_stride + (size_t)v;
-  if (a.out_dtype == DT_F32) ((float*)a.out_logits)[i] = val;
-  else if (a.out_dtype == DT_BF16) ((__bf16*)a.out_logits)[i] = (__bf16)val;
-  else ((_Float16*)a.out_logits)[i] = (_Float16)val;
-}
-
-template <int WT>
-__device__ __forceinline__ f32x4_t mfma16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
-  if constexpr (WT == DT_BF16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  }
-}
-
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-// v_mfma_f32_32x32x16_bf16: lane l holds A row (l & 31) and B column (l & 31)
-// at k = 8 (l >> 5) .. +7; D element e of lane l is row 8 (e >> 2) +
-// 4 (l >> 5) + (e & 3), column l & 31.  Twice the work of a 16x16x32 in
-// about the same issue time on gfx950 (measured ~2.2 vs ~1.25 PFLOP/s).
-__device__ __forceinline__ f32x16_t mfma32x32x16_bf16(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                 0, 0, 0);
-}
-
-__device__ __forceinline__ float apply_cast(float v, int rc) {
-  if (rc == 1) return round_bf16(v);
-  if (rc == 2) return round_f16(v);
-  return v;
-}
-
-__device__ __forceinline__ uint32_t bf16_bits_rne(float v) {
-  uint32_t u = __float_as_uint(v);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x40u;
-  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
-
-// rounds v to element type dt (f32: unchanged)
-__device__ __forceinline__ float round_to_dtype(float v, int dt) {
-  return apply_cast(v, dt == DT_BF16 ? 1 : dt == DT_F16 ? 2 : 0);
-}
-
-// Final RMSNorm of the LM-head prologue, as layers.py:22-29 followed by the
-// activation cast of model.py:758-760: with ss = sum of x^2 over the row (fp32),
-//   y = x * (1 / sqrt(ss / H + eps)) * (1 + w), rounded to the hidden's own type
-// (rms_norm's output.astype(input_dtype)) and then to the activation type.
-__device__ __forceinline__ float prenorm_inv(const LmArgs& a, float ss) {
-  return 1.0f / sqrtf(ss / (float)a.H + a.eps);
-}
-__device__ __forceinline__ float prenorm_apply_w(const LmArgs& a, float x, float inv, float w) {
-  const float y = (x * inv) * (1.0f + w);
-  return round_to_dtype(round_to_dtype(y, a.hidden_dtype), a.act_dtype);
-}
-__device__ __forceinline__ float prenorm_apply(const LmArgs& a, float x, float inv, int k) {
-  return prenorm_apply_w(a, x, inv, load_as_f32(a.norm_w, a.norm_dtype, (size_t)k));
-}
-
-__device__ __forceinline__ uint32_t f16_bits(float v) {
-  _Float16 h = (_Float16)v;
-  uint16_t b;
-  __builtin_memcpy(&b, &h, 2);
-  return b;
-}
-
-// Block-wide max of per-(wave, row) keys held in LDS, then one atomic per row.
-// Each thread waits for its atomics to be performed (their returned values
-// feed an opaque use) before the block barrier, so the ticket taken after the
-// barrier is ordered after every max of the block -- no release fence, which
-// on gfx950 writes back and invalidates the XCD's L2.
-template <int WAVES, int BP>
-__device__ __forceinline__ void block_commit(unsigned long long* red, int B,
-                                             unsigned long long* row_keys) {
-  __syncthreads();
-  for (int b = threadIdx.x; b < B; b += blockDim.x) {
-    unsigned long long m = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) m = max_u64(m, red[w * BP + b]);
-    if (m) (void)after(atomicMax(&row_keys[b], m));
-  }
-}
-
-// Last block to arrive converts the per-row keys into ids and re-zeroes the
-// accumulators and the ticket counter for the next call.
-__device__ __forceinline__ void finish_rows(unsigned long long* row_keys, unsigned int* counter,
-                                            int B, int32_t* out_ids, float* out_best) {
-  __shared__ int s_last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned int t = ticket_add(counter);
-    s_last = (t == gridDim.x - 1);
-  }
-  __syncthreads();
-  if (!s_last) return;
-  for (int b = threadIdx.x; b < B; b += blockDim.x) {
-    unsigned long long k =
-        __hip_atomic_load(&row_keys[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    out_ids[b] = (int32_t)(~(uint32_t)k);
-    if (out_best) out_best[b] = unord_f32((uint32_t)(k >> 32));
-    __hip_atomic_store(&row_keys[b], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Scores N consecutive vocabulary entries v0.. of one batch row (raw fp32
-// dots).  Greedy: folds argmax keys into `best`.  Sample: computes the fast
-// approximate scores for all N in one straight-line block (N interleaved
-// Threefry chains) and marks in q[] (scaled logit xq[], approximate score aq[])
-// every entry that can still be the row's exact maximum:
-// |approx - exact| <= d(s) = 1e-4 + 4.8e-7 |s| (hardware log error ~1e-6 on the
-// draw, plus one ulp of the sum), so the exact maximum j has
-// approx_j >= approx_k - d(s_j) - d(s_k) for every k and is queued when it
-// arrives, whatever set of approximate scores `amax` is the maximum of.
-// Magnitudes are clamped so -inf stays -inf; a NaN scaled logit scores +inf.
-template <int MODE, int N>
-__device__ __forceinline__ void score_run(const float (&raw)[N], int v0, int V, int reduce_cast, bool greedy_row,
-                                          bool unit_tp, float tp, const TfKey& key, float& amax,
-                                          unsigned long long& best, bool (&q)[N], float (&xq)[N], float (&aq)[N]) {
-  // one branch per run, not per element: the cast and the bounds are uniform
-  float val[N];
-  if (reduce_cast == 1) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) val[e] = round_bf16(raw[e]);
-  } else if (reduce_cast == 2) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) val[e] = round_f16(raw[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < N; ++e) val[e] = raw[e];
-  }
-  if (MODE == MODE_SAMPLE && !greedy_row) {
-    float xv[N], ap[N];
-    uint32_t bits[N];
-#pragma unroll
-    for (int e = 0; e < N; ++e) xv[e] = val[e];
-    if (!unit_tp) {
-#pragma unroll
-      for (int e = 0; e < N; ++e) xv[e] = val[e] / tp;
-    }
-    uint32_t idx[N];
-#pragma unroll
-    for (int e = 0; e < N; ++e) idx[e] = (uint32_t)(v0 + e);
-    random_bits32_n<N>(key, idx, bits);
-    // NaN only from a NaN logit (the draw is finite); selecting on the sum
-    // keeps the draws unconditional, so the N chains stay one straight block
-#pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const float t = xv[e] + gumbel_fast_from_bits(bits[e]);
-      ap[e] = (t != t) ? INFINITY : t;
-    }
-    // every draw feeds an unconditional select, so none is sunk into a branch.
-    // One threshold per run instead of the per-entry slack: an entry that
-    // passes ap + 2e-4 + 4.8e-7 (|ap| + |am|) >= am has |ap| <= |am| + slack,
-    // so slack <= 2.01e-4 + 9.61e-7 |am| and ap >= am - that bound: the
-    // queued set only grows (the filter before exact rescoring applies the
-    // per-entry test).  am = -inf queues every entry, am = +inf only +inf.
-    const float am = amax;
-    const float thr = am - (2.01e-4f + 9.61e-7f * fminf(fabsf(am), 1e30f));
-    const bool all_in = v0 + N <= V;  // uniform per run except in the last tile
-#pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const bool ok = all_in || v0 + e < V;
-      q[e] = ok && ap[e] >= thr;
-      xq[e] = xv[e];
-      aq[e] = ap[e];
-      amax = fmaxf(amax, ok ? ap[e] : -INFINITY);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < N; ++e)
-      if (v0 + e < V) best = max_u64(best, argmax_key(val[e], (uint32_t)(v0 + e)));
-  }
-}
 
 // ------------------------------------------------------------------ MFMA kernel
 // WT: weight element type (DT_BF16 / DT_F16).  NSPLIT: hidden terms (1, or 3
@@ -825,28 +601,6 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
   finish_rows(a.row_keys, a.counter, B, a.out_ids, a.out_best);
 }
 
-// Packs eight values into NS bf16 B-fragment words per term: NS = 1 rounds
-// each value to bf16 (exact for bf16 activations); NS = 3 splits an fp32 value
-// exactly into three bf16 terms (hi + mid + lo = v: 8 + 8 + 8 significand bits),
-// so that three bf16 x bf16 products, each exact in fp32, give an fp32-accurate dot.
-template <int NS, int KPW>
-__device__ __forceinline__ void split_terms(const float (&v)[8], u32x4_t (&hb)[NS][KPW], int kk) {
-  float r[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) r[e] = v[e];
-#pragma unroll
-  for (int t = 0; t < NS; ++t) {
-    uint32_t bits[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      bits[e] = bf16_bits_rne(r[e]);
-      r[e] = r[e] - __uint_as_float(bits[e] << 16);
-    }
-    hb[t][kk] = u32x4_t{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16), bits[4] | (bits[5] << 16),
-                        bits[6] | (bits[7] << 16)};
-  }
-}
-
 // ------------------------------------------------------------------ LDS-staged MFMA tile kernel
 // bf16 hidden x bf16 W [V, 1024], 3 <= B <= 64.  A block holds GW "GEMM" waves
 // and NB "epilogue" waves.
@@ -1200,8 +954,19 @@ static int launch_tile(const LmArgs& a, hipStream_t stream) {
   // a second epilogue wave per batch tile (sample mode; measured B=32 91 ->
   // 81 us, B=64 125 -> 118 us): two waves per SIMD issue the draws
   constexpr int EPM = (MODE == MODE_SAMPLE && NB >= 2) ? 2 : 1;
-  auto kern = a.prenorm ? lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, true, NS>
-                        : lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, false, NS>;
+  // (bf16 activations without sampling come here only for the fused prologue
+  // of up to kTilePrenormRows rows)
+  constexpr bool kPlain = NS == 3 || MODE == MODE_SAMPLE;
+  constexpr bool kFused = MODE != MODE_LOGITS && (NS == 3 || NB <= 2);
+  static_assert(kPlain || kFused, "some kernel serves the call");
+  if (a.prenorm ? !kFused : !kPlain) return fail(NVJSEL_EINVAL, "launch_tile: no such variant");
+  auto kern = [&]() {
+    if constexpr (kPlain && kFused)
+      return a.prenorm ? lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, true, NS>
+                       : lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, false, NS>;
+    else
+      return lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, kFused, NS>;
+  }();
   int grid = kTileBpc * device_cu_count();
   const int ntiles = (a.V + 15) / 16;
   if (grid > ntiles) grid = ntiles;
@@ -1216,9 +981,13 @@ static int launch_tile(const LmArgs& a, hipStream_t stream) {
 template <int MODE>
 static int dispatch_tile(const LmArgs& a, hipStream_t s) {
   if (a.act_dtype != DT_BF16) return launch_tile<1, kTileW1, MODE, 3>(a, s);
-  if (a.B <= 16) return launch_tile<1, kTileW1, MODE, 1>(a, s);
-  if (a.B <= 32) return launch_tile<2, kTileW2, MODE, 1>(a, s);
-  return launch_tile<4, kTileW4, MODE, 1>(a, s);
+  if constexpr (MODE == MODE_LOGITS) return fail(NVJSEL_EINVAL, "dispatch_tile: bf16 logits take the staged GEMM");
+  else {
+    if (a.B <= 16) return launch_tile<1, kTileW1, MODE, 1>(a, s);
+    if (MODE != MODE_SAMPLE || a.B <= 32) return launch_tile<2, kTileW2, MODE, 1>(a, s);
+    if constexpr (MODE == MODE_SAMPLE) return launch_tile<4, kTileW4, MODE, 1>(a, s);
+  }
+  return NVJSEL_EINVAL;
 }
 
 // ------------------------------------------------------------------ blocked GEMM, 64 < B <= 256
@@ -1919,14 +1688,12 @@ static size_t lm_ws_keys_bytes(int batch) { return align_up((size_t)batch * 8, 2
 static size_t lm_ws_small_bytes(int batch) {
   return batch <= 0 ? 0 : lm_ws_keys_bytes(batch) + 256;
 }
-// [V, H] bf16: the GEMM above 64 rows; where the tile kernel serves the shape
-// (H = 1024) above 128 rows (greedy / logits) and, sampling, at 129-160 rows
-// and above 192 -- elsewhere its 64-row passes are faster (one box: B = 96
-// 157 vs 168 us greedy, 182 vs 245 us sampled; sampled B = 144 / 160 264 /
-// 270 us in the GEMM against 270-279 / 280-285 in three tile passes, B = 176
-// / 192 296-298 / 300 against 318 / 323)
-static constexpr int kGemmMinBatch = 64, kGemmMinBatchTile = 128, kGemmMinBatchTileSample = 192;
-static constexpr int kGemmBandSample = 160;  // sampling: the GEMM also at kGemmMinBatchTile < B <= this
+// [V, H] bf16 sampling in the blocked GEMM: above 192 rows, and 129-160 (one
+// box, H = 1024: B = 144 / 160 264 / 270 us in the GEMM against 270-279 /
+// 280-285 in three tile passes, B = 176 / 192 296-298 / 300 against 318 / 323)
+static constexpr int kGemmMinBatchTileSample = 192;
+static constexpr int kGemmBandSample = 160;
+static constexpr int kTilePrenormRows = 32;  // bf16 activations: the fused prologue of the tile kernel up to here
 static constexpr int kGemm3MinBatch = 32, kGemm3MinBatchSample = 32;  // f32 activations (three-term GEMM)
 // [H, V] weights: the GEMM above 8 rows for bf16 activations (V = 248k, up
 // to 64 rows in the narrow layout: ~94-98 us greedy, ~113-143 us sampled,
@@ -2068,20 +1835,39 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
     if (nsplit == 3 && tiles > 1) tiles = 1;
     chunk = tiles * 16;
   }
-  const bool tile = !gemv && tile_shape;
-  // blocked GEMM: 64 < B, bf16 activations, one pass over W per 256 rows (greedy, logits and Gumbel sampling)
-  // (sample mode packs vocabulary ids into 25 bits of its queue entries).
-  // [H, V] weights (transposing LDS reads): from 9 rows (bf16), 25 (fp32);
-  // the [H, V] streaming kernel takes 8 rows per pass over W
+  // Staged GEMM on direct LDS loads (lm_head_ring.hip; 16-bit weight and
+  // activations of one type).  Greedy and logits above the GEMV's rows: H =
+  // 1024, V = 248k, B = 16 / 64 / 100 / 256 76 / 78 / 88 / 136 us against 78 /
+  // 81 / 158 / 177 in 64-row tile passes and the blocked GEMM; logits B = 64 /
+  // 80 / 256 102 / 118 / 206 against 149 / 240 / 273; H = 2560, V = 152k, B =
+  // 16 / 64 120 / 134 against 259 / 1010 in the straight-to-registers kernel.
+  // With the norm in the call (a prologue and a zeroing launch, ~11 us) the
+  // tile kernel's fused prologue stays up to 32 rows (85-88 us; 64 rows 100
+  // against 89).  Sampling: wherever the tile kernel does not take the shape,
+  // up to 128 rows per pass; where it does at 65-128 rows (B = 80 / 128 156 /
+  // 183 us against 177-185 / 202-209 in tile passes; B = 64 117-123 against
+  // 103-106) -- above 128 rows the blocked GEMM's single pass is faster (B =
+  // 144 / 256 264 / 340 against 278 / 377), but for the band it leaves.
+  const bool ring_ok = layout == NVJSEL_W_VH && aligned && weight_dtype != NVJSEL_F32 && eff_dtype == weight_dtype &&
+                       (H % 64) == 0 && (prenorm || (((uintptr_t)hidden) & 15) == 0) &&
+                       (mode != MODE_SAMPLE || V < (1 << 25));
+  const bool ring = !gemv && ring_ok &&
+                    (mode != MODE_SAMPLE ? !(prenorm && tile_shape && batch <= kTilePrenormRows)
+                     : tile_shape        ? batch > 64 && batch <= kRingSampleRows
+                                         : batch <= kRingSampleRows || weight_dtype == NVJSEL_F16);
+  const bool tile = !gemv && !ring && tile_shape;
+  // blocked GEMM: sampling bf16 activations on [V, H] above 128 rows (H =
+  // 1024: at 129-160 and above 192), one pass over W per 256 rows (sample
+  // mode packs vocabulary ids into 25 bits of its queue entries); [H, V]
+  // weights (transposing LDS reads) from 9 rows, every mode; the [H, V]
+  // streaming kernel takes 8 rows per pass over W
   const bool hv_gemm_ok = layout == NVJSEL_W_HV && weight_dtype == NVJSEL_BF16 && aligned && (V % 8) == 0;
   const bool gemm_ok = (bf16_mfma || hv_gemm_ok) && (H % (2 * kGemmKC)) == 0 &&
                        (prenorm || (((uintptr_t)hidden) & 15) == 0) && (mode != MODE_SAMPLE || V < (1 << 25));
-  const bool gemm = gemm_ok && eff_dtype == NVJSEL_BF16 &&
-                    (batch > (hv_gemm_ok ? (mode == MODE_SAMPLE ? kGemmHvMinBatchSample : kGemmHvMinBatch)
-                              : !tile    ? kGemmMinBatch
-                                         : (mode == MODE_SAMPLE ? kGemmMinBatchTileSample : kGemmMinBatchTile)) ||
-                     (tile && !hv_gemm_ok && mode == MODE_SAMPLE && batch > kGemmMinBatchTile &&
-                      batch <= kGemmBandSample));
+  const bool gemm = gemm_ok && !ring && eff_dtype == NVJSEL_BF16 &&
+                    (hv_gemm_ok ? batch > (mode == MODE_SAMPLE ? kGemmHvMinBatchSample : kGemmHvMinBatch)
+                                : mode == MODE_SAMPLE && batch > kRingSampleRows &&
+                                      (!tile || batch > kGemmMinBatchTileSample || batch <= kGemmBandSample));
   // f32 activations: the same one-pass GEMM on three bf16 terms per value,
   // per 256-row pass at V = 248k ~460 us (greedy) / ~550-620 us (sampling),
   // ~345-370 / ~475 us for 65-192 rows (padding waves idle), ~180 / ~215 us
@@ -2107,7 +1893,8 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
                      (hv_gemm_ok ? batch > (mode == MODE_SAMPLE ? kGemm3HvMinBatchSample : kGemm3HvMinBatch)
                       : mode == MODE_SAMPLE ? batch > kGemm3MinBatchSample
                                             : batch > kGemm3MinBatch);
-  const bool fused_prenorm = prenorm && !gemm && !gemm3 && !mix3 && (gemv || tile);
+  const bool fused_prenorm = prenorm && !gemm && !gemm3 && !mix3 &&
+                             (gemv || (tile && (eff_dtype != NVJSEL_BF16 || batch <= kTilePrenormRows)));
   if (prenorm && !fused_prenorm) {
     LmArgs p{};
     p.hidden = hidden;
@@ -2127,6 +1914,7 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   if (gemv) chunk = 0;
   if (hv) chunk = 8;
   if (gemm || gemm3) chunk = kGemmBB;
+  if (ring) chunk = mode == MODE_SAMPLE ? kRingSampleRows : kRingRows;
   auto by_mode = [&](auto fn) -> int {
     if (mode == MODE_GREEDY) return fn(std::integral_constant<int, MODE_GREEDY>{});
     if (mode == MODE_SAMPLE) return fn(std::integral_constant<int, MODE_SAMPLE>{});
@@ -2162,9 +1950,13 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
     a.out_dtype = lo.dtype;
     a.out_stride = lo.stride;
     int rc;
-    if (gemm) {
+    if (ring) {
+      rc = launch_ring(mode, a, s);
+    } else if (gemm) {
       rc = by_mode([&](auto M) {
-        return hv_gemm_ok ? launch_gemm<decltype(M)::value, 1, true>(a, s) : launch_gemm<decltype(M)::value, 1, false>(a, s);
+        if (hv_gemm_ok) return launch_gemm<decltype(M)::value, 1, true>(a, s);
+        if constexpr (decltype(M)::value == MODE_SAMPLE) return launch_gemm<MODE_SAMPLE, 1, false>(a, s);
+        return fail(NVJSEL_EINVAL, "lm_head: [V, H] bf16 greedy / logits take the staged GEMM");
       });
     } else if (g3) {
       rc = by_mode([&](auto M) {

@@ -1,0 +1,109 @@
+"""GPU: the staged LM-head GEMM on direct LDS loads (csrc/lm_head_ring.hip)
+at the edges of its tiles, against the oracle: batch rows around each row
+count it is built for, one to several K stages (H = 64 has one, 192 three:
+fewer and more than the ring's slots), vocabularies of one partial tile, of
+more blocks than rows, and of two tiles per block with a remainder
+(V > 256 x 256), bf16 and f16."""
+import numpy as np
+import pytest
+import torch
+
+import nvjsel
+from oracle import selection as sel
+from tests.gpu_helpers import check_fused_sampled, check_greedy, engine_keys, keys_tensor
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, 64, 5), (31, 192, 257), (33, 64, 66000), (64, 320, 2055), (65, 128, 66000), (128, 192, 4099),
+          (129, 64, 70001), (256, 192, 1000), (257, 64, 300)]
+
+
+def _inputs(B, H, V, dt, seed=0):
+    rng = np.random.default_rng(B * 1009 + H + V + seed)
+    h = torch.from_numpy(rng.standard_normal((B, H)).astype(np.float32)).cuda().to(dt)
+    w = torch.from_numpy((rng.standard_normal((V, H)) * 0.3).astype(np.float32)).cuda().to(dt)
+    z = sel.lm_head_logits(h.float().cpu().numpy(), w.float().cpu().numpy())
+    return rng, h, w, z, (1 if dt == torch.bfloat16 else 2)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,V", SHAPES)
+def test_greedy_and_logits(B, H, V, dt):
+    _, h, w, z, rc = _inputs(B, H, V, dt)
+    ids, best = nvjsel.lm_head_greedy_top1_hip(h, w, weight_layout="vh", return_best=True)
+    logits = nvjsel.lm_head_logits_hip(h, w, weight_layout="vh")
+    torch.cuda.synchronize()
+    check_greedy(ids.cpu().numpy(), z, rc, f"ring greedy {dt} {B} {H} {V}")
+    got = logits.float().cpu().numpy().astype(np.float64)
+    # fp32 sums of H products (H 2^-24 sum |h w| <= H 2^-24 |h| |w|) and one
+    # rounding to the 16-bit type (half an ulp: 2^-9 bf16, 2^-12 f16)
+    hn = np.linalg.norm(h.float().cpu().numpy(), axis=1)[:, None]
+    wn = np.linalg.norm(w.float().cpu().numpy(), axis=1)[None, :]
+    tol = H * 2.0 ** -24 * hn * wn * 2 + np.abs(z) * (2.0 ** -8 if rc == 1 else 2.0 ** -11) + 1e-7
+    assert (np.abs(got - z) <= tol).all()
+    # the winning logit is the row's largest stored logit, at its first index
+    np.testing.assert_array_equal(best.cpu().numpy(), logits.float().max(dim=1).values.cpu().numpy())
+    np.testing.assert_array_equal(ids.cpu().numpy().reshape(-1), got.argmax(axis=1))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,V", [s for s in SHAPES if s[0] <= 128 or s[0] == 257])
+def test_sample(B, H, V, dt):
+    rng, h, w, z, rc = _inputs(B, H, V, dt, 1)
+    T = [float(x) for x in rng.choice([0.0, 0.3, 0.7, 1.0, 1.7], B)]
+    keys = engine_keys(B, 7)
+    ids = nvjsel.lm_head_sample_token_ids(h, w, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                          weight_layout="vh")
+    torch.cuda.synchronize()
+    namb = check_fused_sampled(ids.cpu().numpy(), z, T, keys, rc, f"ring sample {dt} {B} {H} {V}")
+    assert namb <= max(2, B // 8)
+
+
+@pytest.mark.parametrize("reduce_cast", [0, 1])
+def test_ties_nan_and_infinities(reduce_cast):
+    """First index among equal rounded logits, first NaN, +inf and all -inf
+    rows; the unrounded comparison too."""
+    B, H, V = 40, 64, 66000
+    rng = np.random.default_rng(5)
+    h = np.zeros((B, H), np.float32)
+    h[:, 0] = 1.0
+    w = np.zeros((V, H), np.float32)
+    w[:, 0] = rng.integers(-40, 40, V) / 8.0  # many exact ties
+    w[300, 0], w[65999, 0] = 7.0, 7.0
+    big = 3.0e38
+    h[1, 1] = h[1, 2] = big  # row 1: inf - inf = NaN at 777 and 65900, +inf at 5
+    w[[777, 65900], 1], w[[777, 65900], 2] = big, -big
+    w[5, 1] = big
+    h[2] = 0.0
+    h[2, 3] = big  # row 2: -inf everywhere
+    w[:, 3] = -big
+    hb = torch.from_numpy(h).cuda().to(torch.bfloat16)
+    wb = torch.from_numpy(w).cuda().to(torch.bfloat16)
+    ids = nvjsel.lm_head_greedy_top1_hip(hb, wb, weight_layout="vh", reduce_cast=reduce_cast).cpu().numpy().reshape(-1)
+    assert ids[0] == 300 and (ids[3:] == 300).all()
+    assert ids[2] == 0
+    assert ids[1] == 777
+
+
+def test_sample_extreme_temperatures_and_nan():
+    """Tiny and huge temperatures (products with 1 / T' out of the float range
+    are divided instead), a NaN temperature and a NaN logit row."""
+    B, H, V = 80, 64, 3001
+    rng = np.random.default_rng(9)
+    h = rng.standard_normal((B, H)).astype(np.float32)
+    w = (rng.standard_normal((V, H)) * 0.3).astype(np.float32)
+    hb = torch.from_numpy(h).cuda().to(torch.bfloat16)
+    wb = torch.from_numpy(w).cuda().to(torch.bfloat16)
+    T = [float(x) for x in rng.choice([1e-7, 1e-3, 0.5, 50.0, 1e30], B)]
+    keys = engine_keys(B, 3)
+    ids = nvjsel.lm_head_sample_token_ids(hb, wb, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                          weight_layout="vh").cpu().numpy()
+    z = sel.lm_head_logits(hb.float().cpu().numpy(), wb.float().cpu().numpy())
+    check_fused_sampled(ids, z, T, keys, 1, "ring sample extreme T")
+    hb[4, 0] = float("nan")
+    T[9] = float("nan")
+    ids = nvjsel.lm_head_sample_token_ids(hb, wb, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                          weight_layout="vh").cpu().numpy()
+    assert ids[4] == 0 and ids[9] == 0  # every score a NaN: the first
+    ok = [b for b in range(B) if b not in (4, 9)]
+    check_fused_sampled(ids[ok], z[ok], [T[b] for b in ok], keys[ok], 1, "ring sample beside NaN rows")
