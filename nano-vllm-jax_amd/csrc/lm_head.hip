@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(kGemvWaves * 64) lm_head_gemv_kernel(LmArgs a)
 }
 
 // ------------------------------------------------------------------ [H, V] streaming kernel
-// Weight stored [H, V] bf16, vocabulary contiguous: the reference's
+// Weight stored [H, V] bf16 or f16 (WT), vocabulary contiguous: the reference's
 // materialised lm_head operand (nanovllm_jax/load_weights.py:256-258; the
 // layout lm_head_triton.py:51-55 reads), B <= 8, activations of any dtype
 // (fp32 activations multiply exactly: every product and sum is fp32).
@@ -454,7 +454,12 @@ __global__ void __launch_bounds__(kGemvWaves * 64) lm_head_gemv_kernel(LmArgs a)
 // KU rows are in flight per wave; acc[b][c] += h[b][k] * W[k][col + c] in
 // fp32, with h broadcast from LDS.  The slices' partial sums meet in LDS,
 // summed in slice order, and each thread then scores two columns of every row.
-template <int NB, int WAVES, int MODE, bool DOTP>
+// Any V >= 8: rows start at any element, so the loads are 16 bytes from any
+// element address (one instruction; V = 50,257, H = 768, B = 4 sampled 1700 ->
+// 23 us against one thread per column).  A group that ends past its row reads on
+// into the next one (those columns are never scored); in the last row it is
+// loaded from V - 8 and moved down.
+template <int WT, int NB, int WAVES, int MODE, bool DOTP>
 __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
   // DOT (bf16 hidden, a k-slice of even length): the hidden sits in LDS as
   // bf16 pairs (k, k+1) and each pair of W rows is packed per column with
@@ -469,7 +474,8 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int H = a.H, V = a.V, B = a.B;
   const int vb = blockIdx.x * STRIP;
-  const int col = min(vb + lane * 8, V - 8);  // clamped loads past the row end (V % 8 == 0)
+  const int col = vb + lane * 8 < V ? vb + lane * 8 : V - 8;  // groups wholly past the row end: any columns
+  const int over = max(col - (V - 8), 0);  // elements of the group past the row end
   if constexpr (DOT) {
     uint32_t* lds_p = (uint32_t*)lds_f;  // [H / 2][NB] bf16 pairs
     const uint16_t* hs = (const uint16_t*)a.hidden;
@@ -512,7 +518,8 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
           const int k = min(k0 + j * KU + u, k1 - 1);
-          ring[decltype(S)::value][u] = stream_load((const u32x4_t*)(W + (size_t)k * V + col));
+          const int c = k == H - 1 ? col - over : col;
+          ring[decltype(S)::value][u] = __builtin_nontemporal_load((const u32x4_any_t*)(W + (size_t)k * V + c));
         }
         __builtin_amdgcn_sched_barrier(0);
       },
@@ -522,7 +529,8 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
           for (int u = 0; u < KU; u += 2) {
             const int k = k0 + i * KU + u;
             if (k >= k1) continue;  // wave-uniform; the slice length is even
-            const u32x4_t w0 = ring[decltype(S)::value][u], w1 = ring[decltype(S)::value][u + 1];
+            u32x4_t w0 = ring[decltype(S)::value][u], w1 = ring[decltype(S)::value][u + 1];
+            if (k + 1 == H - 1) w1 = shift_down8(w1, over);  // (H is even)
             const uint32_t q0[4] = {w0.x, w0.y, w0.z, w0.w}, q1[4] = {w1.x, w1.y, w1.z, w1.w};
             uint32_t wp[8];  // column c: (W[k][c], W[k+1][c]) as a bf16 pair
 #pragma unroll
@@ -545,13 +553,14 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
         for (int u = 0; u < KU; ++u) {
           const int k = k0 + i * KU + u;
           if (k >= k1) continue;  // wave-uniform (last step of the slice)
-          const u32x4_t w = ring[decltype(S)::value][u];
+          u32x4_t w = ring[decltype(S)::value][u];
+          if (k == H - 1) w = shift_down8(w, over);
           const uint32_t q[4] = {w.x, w.y, w.z, w.w};
           float wf[8];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            wf[2 * e] = __uint_as_float(q[e] << 16);
-            wf[2 * e + 1] = __uint_as_float(q[e] & 0xFFFF0000u);
+            wf[2 * e] = WT == DT_BF16 ? __uint_as_float(q[e] << 16) : f16_to_f32((uint16_t)(q[e] & 0xFFFFu));
+            wf[2 * e + 1] = WT == DT_BF16 ? __uint_as_float(q[e] & 0xFFFF0000u) : f16_to_f32((uint16_t)(q[e] >> 16));
           }
           const float* hk = lds_f + k * NB;
 #pragma unroll
@@ -1114,7 +1123,11 @@ __device__ __forceinline__ void gemm_finish_rows(const LmArgs& a, unsigned long 
 // NARROW: B <= 64; each wave owns 32 vocabulary rows x the 64 batch rows
 // (instead of 128 x 64 of one batch quarter), so all 8 waves multiply and,
 // in sample mode, draw.
-template <int MODE, int BV, int NS, int KC, bool HV, bool PART, bool NARROW>
+// WT: weight (and NS = 1: hidden) element type.  [H, V] rows start at any
+// element (V >= 8): 16-byte loads from element addresses; a group that ends
+// past its row reads on into the next one (columns masked where they could
+// win), in the last row it is loaded from V - 8 and moved down as it is stored.
+template <int WT, int MODE, int BV, int NS, int KC, bool HV, bool PART, bool NARROW>
 __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a) {
   constexpr int Q = KC / 8;  // 8-element columns per row and stage
   static_assert(!(PART && NARROW), "one batch layout");
@@ -1190,6 +1203,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
   // path has the same loads in flight and each LDS store waits for exactly
   // its own stage.
   u32x4_t RA[2][PA], RB[2][PB][HB];
+  int over[2][PA] = {};  // HV: places each piece moves down
   auto stage_of = [&](int st, int& v0, int& kc) NVJSEL_INLINE {
     st = st < S ? st : S - 1;
     const int t = st / nkc;
@@ -1203,10 +1217,10 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
       if constexpr (HV) {
-        // groups past the row end re-read the last group (V % 8 == 0); their
-        // columns are masked where they could win
-        const int v = min(v0 + aq[i] * 8, V - 8);
-        RA[e][i] = *(const u32x4_t*)(W + (size_t)(kc * KC + arow[i]) * V + v);
+        const int k = kc * KC + arow[i];
+        const int v = v0 + aq[i] * 8 < V ? v0 + aq[i] * 8 : V - 8;
+        over[e][i] = k == H - 1 ? max(v - (V - 8), 0) : 0;
+        RA[e][i] = *(const u32x4_any_t*)(W + (size_t)k * V + (v - over[e][i]));
       } else {
         const int v = min(v0 + arow[i], V - 1);
         RA[e][i] = *((const u32x4_t*)(W + (size_t)v * H + kc * KC) + aq[i]);
@@ -1226,7 +1240,12 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
   auto lstore = [&](auto set, auto buf) NVJSEL_INLINE {
     constexpr int e = decltype(set)::value, f = decltype(buf)::value;
 #pragma unroll
-    for (int i = 0; i < PA; ++i) As[f][aslot[i]] = RA[e][i];
+    for (int i = 0; i < PA; ++i) {
+      if constexpr (HV) {
+        if (__any(over[e][i])) RA[e][i] = shift_down8(RA[e][i], over[e][i]);
+      }
+      As[f][aslot[i]] = RA[e][i];
+    }
     if (XT < NT && tid >= XT) return;  // (wave-uniform)
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
@@ -1289,7 +1308,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
 #pragma unroll
         for (int t = 0; t < NS; ++t)
 #pragma unroll
-          for (int tb = 0; tb < 2; ++tb) acc[tv][tb] = mfma32x32x16_bf16(af, bf[t][tb], acc[tv][tb]);
+          for (int tb = 0; tb < 2; ++tb) acc[tv][tb] = mfma32x32x16<WT>(af, bf[t][tb], acc[tv][tb]);
       }
     }
   };
@@ -1493,7 +1512,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
 // 185 us at B = 256, V = 248320) or 128 (4 waves, two blocks per CU: 195 us)
 static constexpr int kGemmBV = 256;
 static constexpr int kGemmBpc = 256 / kGemmBV;  // blocks per CU of the blocked GEMM
-template <int MODE, int NS, bool HV>
+template <int WT, int MODE, int NS, bool HV>
 static int launch_gemm(const LmArgs& a, hipStream_t stream) {
   const int ntiles = (a.V + kGemmBV - 1) / kGemmBV;
   int grid = kGemmBpc * device_cu_count();
@@ -1503,12 +1522,21 @@ static int launch_gemm(const LmArgs& a, hipStream_t stream) {
   // <= 64 rows take the tile kernel; its 64-row f32 stages leave room for
   // K stages of 32 in sample mode)
   constexpr bool kNarrow = HV || NS == 3;
-  if (kNarrow && a.B <= 64)
-    hipLaunchKernelGGL((lm_head_gemm_kernel<MODE, kGemmBV, NS, kGemmKC, HV, false, kNarrow>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
-  else if (a.B <= kGemmBB - 64)
-    hipLaunchKernelGGL((lm_head_gemm_kernel<MODE, kGemmBV, NS, KC, HV, true, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
-  else
-    hipLaunchKernelGGL((lm_head_gemm_kernel<MODE, kGemmBV, NS, KC, HV, false, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+  if constexpr (kNarrow) {
+    if (a.B <= 64) {
+      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, kGemmKC, HV, false, true>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+      NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
+      return NVJSEL_OK;
+    }
+  }
+  if constexpr (WT == DT_F16) {
+    return fail(NVJSEL_EINVAL, "launch_gemm: f16 weights take at most 64 rows");
+  } else {
+    if (a.B <= kGemmBB - 64)
+      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, true, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+    else
+      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, false, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+  }
   NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
   return NVJSEL_OK;
 }
@@ -1732,11 +1760,13 @@ struct LogitsOut {
   long long stride = 0;
 };
 
-template <int NB, int MODE>
+template <int WT, int NB, int MODE>
 static int launch_hv(const LmArgs& a, hipStream_t stream) {
   constexpr int WAVES = 4;  // measured: 4 waves per block beat 8 and 16 at B = 1 and 8
-  const bool dot = kHvDot && a.hidden_dtype == DT_BF16 && (a.H % (2 * WAVES)) == 0;
-  auto kern = dot ? lm_head_hv_kernel<NB, WAVES, MODE, true> : lm_head_hv_kernel<NB, WAVES, MODE, false>;
+  auto kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, false>;
+  if constexpr (WT == DT_BF16) {
+    if (kHvDot && a.hidden_dtype == DT_BF16 && (a.H % (2 * WAVES)) == 0) kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, true>;
+  }
   const size_t lds = hv_lds_bytes(NB, a.H);
   if (lds > 48 * 1024)
     NVJSEL_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1745,12 +1775,17 @@ static int launch_hv(const LmArgs& a, hipStream_t stream) {
   return NVJSEL_OK;
 }
 
+template <int WT, int MODE>
+static int dispatch_hv_type(const LmArgs& a, hipStream_t s) {
+  if (a.B == 1) return launch_hv<WT, 1, MODE>(a, s);
+  if (a.B == 2) return launch_hv<WT, 2, MODE>(a, s);
+  if (a.B <= 4) return launch_hv<WT, 4, MODE>(a, s);
+  return launch_hv<WT, 8, MODE>(a, s);
+}
+
 template <int MODE>
 static int dispatch_hv(const LmArgs& a, hipStream_t s) {
-  if (a.B == 1) return launch_hv<1, MODE>(a, s);
-  if (a.B == 2) return launch_hv<2, MODE>(a, s);
-  if (a.B <= 4) return launch_hv<4, MODE>(a, s);
-  return launch_hv<8, MODE>(a, s);
+  return a.weight_dtype == DT_BF16 ? dispatch_hv_type<DT_BF16, MODE>(a, s) : dispatch_hv_type<DT_F16, MODE>(a, s);
 }
 
 static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const void* weight,
@@ -1821,8 +1856,8 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   const bool gemv = gemv_shape && (mode == MODE_SAMPLE
                                        ? batch <= 2 && (!tile_shape || (batch == 1 && eff_dtype != NVJSEL_BF16))
                                        : batch <= 2 || (batch <= 4 && eff_dtype != NVJSEL_BF16));
-  // [H, V] bf16 streaming kernel, up to 8 rows per launch
-  const bool hv = layout == NVJSEL_W_HV && weight_dtype == NVJSEL_BF16 && aligned && (V % 8) == 0 &&
+  // [H, V] 16-bit streaming kernel, up to 8 rows per launch, any V >= 8
+  const bool hv = layout == NVJSEL_W_HV && weight_dtype != NVJSEL_F32 && (((uintptr_t)weight) & 1) == 0 && V >= 8 &&
                   hv_lds_bytes(batch < 8 ? batch : 8, H) + kStaticLdsSlack <= device_max_lds_per_block();
   // rows per launch: LDS holds H * nsplit * rows bf16 values
   int chunk = 0;
@@ -1861,11 +1896,20 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // mode packs vocabulary ids into 25 bits of its queue entries); [H, V]
   // weights (transposing LDS reads) from 9 rows, every mode; the [H, V]
   // streaming kernel takes 8 rows per pass over W
-  const bool hv_gemm_ok = layout == NVJSEL_W_HV && weight_dtype == NVJSEL_BF16 && aligned && (V % 8) == 0;
+  const bool hv_gemm_ok = layout == NVJSEL_W_HV && V >= 8 && (((uintptr_t)weight) & 1) == 0 &&
+                          (weight_dtype == NVJSEL_BF16 || (weight_dtype == NVJSEL_F16 && eff_dtype == NVJSEL_F16));
   const bool gemm_ok = (bf16_mfma || hv_gemm_ok) && (H % (2 * kGemmKC)) == 0 &&
                        (prenorm || (((uintptr_t)hidden) & 15) == 0) && (mode != MODE_SAMPLE || V < (1 << 25));
-  const bool gemm = gemm_ok && !ring && eff_dtype == NVJSEL_BF16 &&
-                    (hv_gemm_ok ? batch > (mode == MODE_SAMPLE ? kGemmHvMinBatchSample : kGemmHvMinBatch)
+  // Its 512-column strips leave CUs idle on a small vocabulary (V = 50,257, H
+  // = 768, 99 blocks: sampled B = 1 / 4 / 8 30 / 36 / 46 us; the GEMM's 197
+  // tiles ~28 at 1-16 rows), and f16 weights have no two-product dot there
+  // (V = 128,256, H = 2048, B = 1 / 8 84 / 142 us against 94)
+  const int hv_gemm_min = (V + 511) / 512 <= device_cu_count() / 2 ? 0
+                          : weight_dtype == NVJSEL_F16             ? 2
+                          : mode == MODE_SAMPLE                    ? kGemmHvMinBatchSample
+                                                                   : kGemmHvMinBatch;
+  const bool gemm = gemm_ok && !ring && eff_dtype == weight_dtype &&
+                    (hv_gemm_ok ? batch > hv_gemm_min
                                 : mode == MODE_SAMPLE && batch > kRingSampleRows &&
                                       (!tile || batch > kGemmMinBatchTileSample || batch <= kGemmBandSample));
   // f32 activations: the same one-pass GEMM on three bf16 terms per value,
@@ -1913,7 +1957,7 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   if (tile) chunk = eff_dtype == NVJSEL_BF16 ? 64 : 16;
   if (gemv) chunk = 0;
   if (hv) chunk = 8;
-  if (gemm || gemm3) chunk = kGemmBB;
+  if (gemm || gemm3) chunk = gemm && weight_dtype == NVJSEL_F16 ? 64 : kGemmBB;
   if (ring) chunk = mode == MODE_SAMPLE ? kRingSampleRows : kRingRows;
   auto by_mode = [&](auto fn) -> int {
     if (mode == MODE_GREEDY) return fn(std::integral_constant<int, MODE_GREEDY>{});
@@ -1954,13 +1998,16 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
       rc = launch_ring(mode, a, s);
     } else if (gemm) {
       rc = by_mode([&](auto M) {
-        if (hv_gemm_ok) return launch_gemm<decltype(M)::value, 1, true>(a, s);
-        if constexpr (decltype(M)::value == MODE_SAMPLE) return launch_gemm<MODE_SAMPLE, 1, false>(a, s);
+        if (hv_gemm_ok)
+          return weight_dtype == NVJSEL_F16 ? launch_gemm<DT_F16, decltype(M)::value, 1, true>(a, s)
+                                            : launch_gemm<DT_BF16, decltype(M)::value, 1, true>(a, s);
+        if constexpr (decltype(M)::value == MODE_SAMPLE) return launch_gemm<DT_BF16, MODE_SAMPLE, 1, false>(a, s);
         return fail(NVJSEL_EINVAL, "lm_head: [V, H] bf16 greedy / logits take the staged GEMM");
       });
     } else if (g3) {
       rc = by_mode([&](auto M) {
-        return hv_gemm_ok ? launch_gemm<decltype(M)::value, 3, true>(a, s) : launch_gemm<decltype(M)::value, 3, false>(a, s);
+        return hv_gemm_ok ? launch_gemm<DT_BF16, decltype(M)::value, 3, true>(a, s)
+                          : launch_gemm<DT_BF16, decltype(M)::value, 3, false>(a, s);
       });
     } else if (gv) {
       rc = by_mode([&](auto M) { return dispatch_gemv<decltype(M)::value>(a, s); });

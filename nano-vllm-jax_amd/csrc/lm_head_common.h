@@ -20,6 +20,16 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));  // a 16-byte load from any element address
+
+// The eight 16-bit elements of w moved down by s places (0 <= s <= 7).
+__device__ __forceinline__ u32x4_t shift_down8(u32x4_t w, int s) {
+  const uint64_t lo = ((uint64_t)w.y << 32) | w.x, hi = ((uint64_t)w.w << 32) | w.z;
+  const int b = 16 * (s & 3);
+  const uint64_t l1 = s & 4 ? hi : lo, h1 = s & 4 ? 0ull : hi;
+  const uint64_t l2 = b ? (l1 >> b) | (h1 << (64 - b)) : l1, h2 = h1 >> b;
+  return u32x4_t{(uint32_t)l2, (uint32_t)(l2 >> 32), (uint32_t)h2, (uint32_t)(h2 >> 32)};
+}
 
 // GREEDY: argmax id per row; SAMPLE: Gumbel-max id per row; LOGITS: the
 // (REDUCE_CAST-rounded) logits themselves, written to out_logits.
@@ -74,13 +84,18 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(u32x4_t a, u32x4_t b, f32x4_t c)
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-// v_mfma_f32_32x32x16_bf16: lane l holds A row (l & 31) and B column (l & 31)
+// v_mfma_f32_32x32x16_bf16 / _f16: lane l holds A row (l & 31) and B column (l & 31)
 // at k = 8 (l >> 5) .. +7; D element e of lane l is row 8 (e >> 2) +
 // 4 (l >> 5) + (e & 3), column l & 31.  Twice the work of a 16x16x32 in
 // about the same issue time on gfx950 (measured ~2.2 vs ~1.25 PFLOP/s).
-__device__ __forceinline__ f32x16_t mfma32x32x16_bf16(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                 0, 0, 0);
+template <int WT>
+__device__ __forceinline__ f32x16_t mfma32x32x16(u32x4_t a, u32x4_t b, f32x16_t c) {
+  if constexpr (WT == DT_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                   0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
+                                                  0, 0);
 }
 
 __device__ __forceinline__ float apply_cast(float v, int rc) {

@@ -83,16 +83,6 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int WT>
-__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
-  if constexpr (WT == DT_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
-                                                  0, 0);
-}
-
 // The smallest float that rounds (to nearest even) to the bf16 value r, not NaN.
 __device__ __forceinline__ float bf16_round_low(float r) {
   uint32_t u = __float_as_uint(r);
@@ -210,8 +200,8 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     for (int tv = 0; tv < TV; ++tv)
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
-        acc[tv][tb] = MODE == MODE_LOGITS ? mfma32<WT>(fb[f][tb], fa[f][tv], acc[tv][tb])
-                                          : mfma32<WT>(fa[f][tv], fb[f][tb], acc[tv][tb]);
+        acc[tv][tb] = MODE == MODE_LOGITS ? mfma32x32x16<WT>(fb[f][tb], fa[f][tv], acc[tv][tb])
+                                          : mfma32x32x16<WT>(fa[f][tv], fb[f][tb], acc[tv][tb]);
     __builtin_amdgcn_sched_barrier(0);
   };
   using I0 = std::integral_constant<int, 0>;
