@@ -275,9 +275,16 @@ __device__ __forceinline__ void split_terms(const float (&v)[8], u32x4_t (&hb)[N
 }
 
 // lm_head_ring.hip: one pass over W for up to kRingRows batch rows (sampling:
-// kRingSampleRows); 16-bit weight [V, H] and hidden of the same type, both
-// 16-byte aligned, H % 64 == 0 (sampling: V < 2^25).
-static constexpr int kRingRows = 256, kRingSampleRows = 128;
+// kRingSampleRows); 16-bit weight [V, H] and hidden of the same type, or bf16
+// weight and f32 hidden (kRingF32Rows), 16-byte aligned, H % 64 == 0
+// (sampling: V < 2^25).
+static constexpr int kRingRows = 256, kRingSampleRows = 128, kRingF32Rows = 64;
 int launch_ring(int mode, const LmArgs& a, hipStream_t stream);
+
+// lm_head_gemm.hip: one pass over W for up to kGemmBB rows; hv: [H, V] weights
+// (16-bit hidden of the same type -- f16 at most 64 rows -- or f32 on bf16),
+// else on bf16 [V, H] bf16 sampling or f32 hidden; H % (2 kGemmKC) == 0.
+static constexpr int kGemmBB = 256, kGemmKC = 32;
+int launch_gemm(int mode, bool hv, const LmArgs& a, hipStream_t stream);
 
 }  // namespace nvjsel

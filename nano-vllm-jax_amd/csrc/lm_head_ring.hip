@@ -1,7 +1,8 @@
 // LM head as a staged GEMM whose operands reach the LDS by direct loads (gfx950).
 //
 // 16-bit weight [V, H] x hidden of the same type, H % 64 == 0, up to 256 batch
-// rows per pass over W (sampling: 128): greedy top-1, dense logits, Gumbel-max.
+// rows per pass over W (sampling: 128), or bf16 weight x f32 hidden, up to 64:
+// greedy top-1, dense logits, Gumbel-max.
 //
 // One block of 8 waves per CU takes an equal, contiguous share of the
 // vocabulary in tiles of 256 rows x all batch rows; K streams in stages of 64.
@@ -28,6 +29,12 @@
 //    small units beside the next tile's stages (B = 64 136 -> 117-123 us, B =
 //    128 224 -> 183); the waves share the rows' maxima through the LDS, so few
 //    entries queue for exact scores.
+//  * f32 hidden (NS = 3): a stage arrives as f32 beside the ring and is split
+//    into three bf16 terms in the middle of the stage before its own (once per
+//    block; through registers, whose waits drained the W stage in flight too,
+//    B = 16 took 99 us against 87).  Fragment reads bound it at 64 rows: 64 x
+//    32 per wave instead of 32 x 64 reads 160 KB per stage instead of 224 (B =
+//    64 126 -> 121 us).
 // H = 1024, V = 248,320, greedy B = 16 / 64 / 128 / 256: 76 / 78 / 90 / 136 us
 // (6.6 / 6.5 / 5.7 / 3.7 TB/s; 956 TFLOP/s at 256) where 64-row passes of the
 // tile kernel and the blocked GEMM took 78 / 81 / 160 / 177.
@@ -39,23 +46,30 @@ namespace nvjsel {
 
 static constexpr int kRingKC = 64;  // K per stage: 128-byte pieces of W rows, whole cache lines
 
-// NBR: batch rows of the block (rows past B repeat row B - 1).
-template <int MODE, int NBR>
+// NBR: batch rows of the block (rows past B repeat row B - 1).  NS: terms per
+// hidden value (3: f32 hidden, each value split exactly into three bf16 terms
+// as it is staged, three products per fragment pair).
+template <int MODE, int NBR, int NS>
 struct RingShape {
+  static_assert(NS == 1 || (NS == 3 && NBR <= 64), "the terms' slots fit the LDS");
   static constexpr bool SMP = MODE == MODE_SAMPLE;
   static constexpr int NW = 8;                        // waves; one block per CU
   static constexpr int BV = 256;                      // vocabulary rows of a block tile
-  static constexpr int TB = NBR <= 32 ? 1 : 2;        // 32-row batch tiles per wave
+  static constexpr int TB = NBR <= 32 || NS == 3 ? 1 : 2;  // 32-row batch tiles per wave
   static constexpr int WB = NBR / (32 * TB);          // waves along the batch
   static constexpr int WV = NW / WB;                  // waves along the vocabulary
   static constexpr int TV = BV / (32 * WV);           // 32-row vocabulary tiles per wave
   // ring slots: W stages come from HBM, hidden stages from L2
-  static constexpr int RW = SMP ? (NBR <= 64 ? 3 : 2) : NBR <= 32 ? 4 : 3;
-  static constexpr int RX = SMP ? 2 : NBR <= 32 ? 4 : NBR <= 128 ? 3 : 2;
-  static constexpr int LDS_RING = (RW * BV + RX * NBR) * kRingKC * 2;
-  // sample mode: queue entries per wave (12 B each), the rows' shared maxima
-  static constexpr int QC = NBR <= 32 ? 512 : NBR <= 64 ? 384 : 512;
-  static constexpr int LDS_QUEUE = SMP ? NW * (QC * 12 + 64 * TB * 8) + NBR * 4 : 0;
+  static constexpr int RW = NS == 3 ? (SMP && NBR == 64 ? 2 : 3) : SMP ? (NBR <= 64 ? 3 : 2) : NBR <= 32 ? 4 : 3;
+  static constexpr int RX = NS == 3 || SMP ? 2 : NBR <= 32 ? 4 : NBR <= 128 ? 3 : 2;
+  static constexpr int LDS_RAW = NS == 3 ? NBR * kRingKC * 4 : 0;  // one stage of f32 values
+  static constexpr int LDS_RING = (RW * BV + RX * NS * NBR) * kRingKC * 2 + LDS_RAW;
+  // sample mode: rows scored at a time, queue entries per wave (12 B each), and
+  // per batch row the block's largest approximate score and best exact key
+  static constexpr int RUN = 4;
+  static constexpr int QC = NS == 3 ? 320 : NBR == 64 ? 480 : 512;
+  static constexpr int LDS_QUEUE = SMP ? NW * QC * 12 + NBR * 12 : 0;
+  static_assert(QC >= 64 * RUN, "room for one unit");
   static_assert(LDS_RING + LDS_QUEUE <= 160 * 1024, "fits the LDS");
 };
 
@@ -92,19 +106,40 @@ __device__ __forceinline__ float bf16_round_low(float r) {
   return __uint_as_float((u & 0x80000000u) ? u + half : u - half);
 }
 
+// The next of the three bf16 terms of four f32 values (round to nearest even),
+// which leave the remainders: hi + mid + lo = v exactly (8 + 8 + 8 bits).
+__device__ __forceinline__ uint2 next_term(float (&v)[4]) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  uint32_t o[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{v[2 * j], v[2 * j + 1]}), bf16x2_t));
+    v[2 * j] = v[2 * j] - __uint_as_float(o[j] << 16);
+    v[2 * j + 1] = v[2 * j + 1] - __uint_as_float(o[j] & 0xFFFF0000u);
+  }
+  return uint2{o[0], o[1]};
+}
+
+// This wave's direct loads but the newest N have landed.
+template <int N>
+__device__ __forceinline__ void wave_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // rows: vocabulary rows per block (a multiple of 8).
-template <int WT, int MODE, int NBR>
+template <int WT, int MODE, int NBR, int NS>
 __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
-  using S = RingShape<MODE, NBR>;
-  constexpr int TV = S::TV, TB = S::TB, WV = S::WV, RW = S::RW, RX = S::RX, NW = S::NW, QC = S::QC;
+  using S = RingShape<MODE, NBR, NS>;
+  constexpr int TV = S::TV, TB = S::TB, WV = S::WV, RW = S::RW, RX = S::RX, NW = S::NW, QC = S::QC, RUN = S::RUN;
   constexpr int BV = S::BV;
-  constexpr int WBYTES = BV * kRingKC * 2, XBYTES = NBR * kRingKC * 2;
+  constexpr int WBYTES = BV * kRingKC * 2, XBYTES = NS * NBR * kRingKC * 2;
   constexpr int WL = WBYTES / (NW * 1024);                              // W loads per wave and stage
   constexpr int XL = XBYTES >= NW * 1024 ? XBYTES / (NW * 1024) : 1;     // hidden loads per wave and stage
   constexpr int XLANES = XBYTES >= NW * 1024 ? 64 : XBYTES / (NW * 16);  // lanes of each
   // loads a wave may leave in flight when stage s starts: those issued after
   // X(s) and W(s) (each stage issues X(s + RX - 1), then W(s + RW - 1))
-  constexpr int LIVE = (RX - 2) * (WL + XL) + (RW > RX ? WL : 0);
+  // (NS = 3: X(s) is split already; W(s + 1) is in flight where RW = 3)
+  constexpr int LIVE = NS == 3 ? (RW - 2) * WL : (RX - 2) * (WL + XL) + (RW > RX ? WL : 0);
   static_assert(RW >= RX && RX >= 2, "W runs at least as far ahead as the hidden");
   constexpr int XRING = RW * WBYTES;  // LDS offset of the hidden's slots
   __shared__ __attribute__((aligned(1024))) char ring[S::LDS_RING + S::LDS_QUEUE];
@@ -153,6 +188,36 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     lx = lx + 1 == RX ? 0 : lx + 1;
     xko = xko + kRingKC * 2 == rowb ? 0u : xko + kRingKC * 2;
   };
+  // NS = 3: the next hidden stage arrives as f32 in `raw`, each thread's 16-byte
+  // pieces (four values) where it reads them back itself, and is split into
+  // the other slot in the middle of a stage
+  constexpr int RL = S::LDS_RAW / (NW * 1024);  // raw loads per wave and stage
+  constexpr int RAW = XRING + RX * XBYTES;
+  auto issue_raw = [&]() NVJSEL_INLINE {
+    const char* src = hidden + 2 * xko;
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      const int p = (i * NW + wave) * 64 + lane;  // row p >> 4, values 4 (p & 15) .. + 3
+      dma16(src, (uint32_t)min(p >> 4, B - 1) * (2 * rowb) + (uint32_t)(p & 15) * 16u,
+            ring0 + (uint32_t)(RAW + (i * NW + wave) * 1024));
+    }
+    xko = xko + kRingKC * 2 == rowb ? 0u : xko + kRingKC * 2;
+  };
+  auto split_raw = [&]() NVJSEL_INLINE {  // (this wave's raw loads have landed)
+    char* dst = ring + XRING + lx * XBYTES;
+    lx ^= 1;
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      const int p = (i * NW + wave) * 64 + lane, row = p >> 4, q = (p & 15) >> 1;
+      const u32x4_t r = *(const u32x4_t*)(ring + RAW + p * 16);
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(r[j]);
+      char* at = dst + row * (kRingKC * 2) + ((q ^ ((row >> 1) & 7)) * 16) + (p & 1) * 8;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) *(uint2*)(at + t * (NBR * kRingKC * 2)) = next_term(v);
+    }
+  };
   auto issue_w = [&]() NVJSEL_INLINE {
     const uint32_t dst = ring0 + (uint32_t)(lw * WBYTES);
     const char* src = wtile + lko;
@@ -182,14 +247,16 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
   // stage barrier too: two register sets, the scheduling barriers keep the
   // reads of the next step ahead of this step's products.
   int cw = 0, cx = 0;  // ring slots of the stage being multiplied
-  u32x4_t fa[2][TV], fb[2][TB];
+  u32x4_t fa[2][TV], fb[2][NS][TB];
   auto read_step = [&](auto set, auto KS) NVJSEL_INLINE {
     constexpr int f = decltype(set)::value, ks = decltype(KS)::value;
     const int col = ((ks * 2 + h) ^ sw) * 16 + c32 * (kRingKC * 2);
     const char* wbuf = ring + cw * WBYTES + wv * TV * 32 * (kRingKC * 2) + col;
     const char* xbuf = ring + XRING + cx * XBYTES + wb * 32 * TB * (kRingKC * 2) + col;
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb) fb[f][tb] = *(const u32x4_t*)(xbuf + tb * 32 * (kRingKC * 2));
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) fb[f][t][tb] = *(const u32x4_t*)(xbuf + (t * NBR + tb * 32) * (kRingKC * 2));
 #pragma unroll
     for (int tv = 0; tv < TV; ++tv) fa[f][tv] = *(const u32x4_t*)(wbuf + tv * 32 * (kRingKC * 2));
     __builtin_amdgcn_sched_barrier(0);
@@ -199,9 +266,11 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
 #pragma unroll
     for (int tv = 0; tv < TV; ++tv)
 #pragma unroll
-      for (int tb = 0; tb < TB; ++tb)
-        acc[tv][tb] = MODE == MODE_LOGITS ? mfma32x32x16<WT>(fb[f][tb], fa[f][tv], acc[tv][tb])
-                                          : mfma32x32x16<WT>(fa[f][tv], fb[f][tb], acc[tv][tb]);
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+          acc[tv][tb] = MODE == MODE_LOGITS ? mfma32x32x16<WT>(fb[f][t][tb], fa[f][tv], acc[tv][tb])
+                                            : mfma32x32x16<WT>(fa[f][tv], fb[f][t][tb], acc[tv][tb]);
     __builtin_amdgcn_sched_barrier(0);
   };
   using I0 = std::integral_constant<int, 0>;
@@ -211,12 +280,19 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
   // one stage; `rest`: the previous stage of the tile left its last step's products
   auto stage = [&](auto rest) NVJSEL_INLINE {
     stage_barrier<LIVE>();
-    issue_x();
+    if constexpr (NS == 3)
+      issue_raw();
+    else
+      issue_x();
     issue_w();
     read_step(I0{}, I0{});
     if constexpr (decltype(rest)::value) multiply(I1{});
     read_step(I1{}, I1{});
     multiply(I0{});
+    if constexpr (NS == 3) {
+      wave_wait<WL>();  // the W stage requested behind the raw values stays in flight
+      split_raw();
+    }
     read_step(I0{}, I2{});
     multiply(I1{});
     read_step(I1{}, I3{});
@@ -228,14 +304,13 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) bo[tb] = bi[tb] = 0u;
   // ---- sample mode: per wave a queue of the entries that may be their row's
-  // maximum (logit, approximate score, vocab << 7 | tb << 6 | lane), the exact
-  // best key of each (lane, tb) row slot, and the block's largest approximate
-  // score of each row (ord_f32), shared by the waves
+  // maximum (logit, approximate score, vocab << 7 | tb << 6 | lane); shared by
+  // the waves, each row's best exact key and largest approximate score (ord_f32)
   float* const qx = (float*)(ring + S::LDS_RING) + wave * QC;
   float* const qa = (float*)(ring + S::LDS_RING) + (NW + wave) * QC;
   uint32_t* const qv = (uint32_t*)(ring + S::LDS_RING) + (2 * NW + wave) * QC;
-  unsigned long long* const qbest = (unsigned long long*)(ring + S::LDS_RING + NW * QC * 12) + wave * 64 * TB;
-  uint32_t* const rowmax = (uint32_t*)(ring + S::LDS_RING + NW * (QC * 12 + 64 * TB * 8)) + wb * 32 * TB + c32;
+  unsigned long long* const rowbest = (unsigned long long*)(ring + S::LDS_RING + NW * QC * 12);  // [NBR]
+  uint32_t* const rowmax = (uint32_t*)(rowbest + NBR) + wb * 32 * TB + c32;
   float tp[TB], rtp[TB], amax[TB];
   bool greedy_row[TB];
   TfKey key[TB];
@@ -252,8 +327,8 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
       key[tb] = b < B ? tf_key(a.keys[2 * b], a.keys[2 * b + 1]) : tf_key(0u, 0u);
       amax[tb] = -INFINITY;
       sbest[tb] = 0ull;
-      qbest[tb * 64 + lane] = 0ull;
-      rowmax[tb * 32] = 0u;  // (ordered before its first use by the stages' barriers)
+      rowbest[wb * 32 * TB + tb * 32 + c32] = 0ull;  // (ordered before their first use by the stages' barriers)
+      rowmax[tb * 32] = 0u;
     }
   }
   // Bound on |approximate - exact| of two scores ap, am together: 1e-4 covers
@@ -295,7 +370,7 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     qcount = nk;
   };
   // exact scores (correctly rounded division, fp64 logs) of the queued entries,
-  // a full wave at a time, folded into the row slots' exact best keys
+  // a full wave at a time, folded into the rows' best keys
   auto flush = [&]() NVJSEL_INLINE {
     for (uint32_t e0 = 0; e0 < qcount; e0 += 64) {  // wave-uniform trip count
       const uint32_t e = e0 + lane;
@@ -314,67 +389,70 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
       }
       const TfKey k2 = tf_key(t1 ? kw[TB - 1][0] : kw[0][0], t1 ? kw[TB - 1][1] : kw[0][1]);
       const uint32_t v = pv >> 7;
-      if (live) atomicMax(&qbest[pv & 127u], argmax_key(qx[e] / (t1 ? tw[TB - 1] : tw[0]) + gumbel_at(k2, v), v));
+      if (live) atomicMax(&rowbest[wb * 32 * TB + (t1 ? 32 : 0) + (sl & 31)],
+                          argmax_key(qx[e] / (t1 ? tw[TB - 1] : tw[0]) + gumbel_at(k2, v), v));
     }
     qcount = 0;
   };
-  // A finished tile's logits wait in `pend` and are scored in units -- four
+  // A finished tile's logits wait in `pend` and are scored in units -- RUN
   // consecutive vocabulary rows of one of the lane's batch rows (D element e:
   // row pv0 + tv * 32 + 8 (e >> 2) + 4 h + (e & 3)) -- spread over the next
   // tile's stages, so that the draws run while W streams; the two waves of a
   // SIMD are half a period apart.  After a unit the row's elements shift
   // down: the indices stay compile-time constants.
-  constexpr int NUNIT = S::SMP ? TV * 4 * TB : 0;
+  constexpr int NUNIT = S::SMP ? TV * (16 / RUN) * TB : 0;
   f32x16_t pend[S::SMP ? TV : 1][TB];
   int pv0 = 0, pvend = 0, punit = NUNIT, credit = 0;
   auto pending = [&]() NVJSEL_INLINE {  // (false: all scored, or only repeats of the tile's last row left)
-    return punit < NUNIT && pv0 + punit / TB * 8 < pvend;
+    return punit < NUNIT && pv0 + (punit / TB * RUN >> 2) * 8 < pvend;
   };
   auto score_row = [&](auto TBI) NVJSEL_INLINE {
     constexpr int tb = decltype(TBI)::value;
-    const int vs = pv0 + punit / TB * 8 + 4 * h;
+    const int e0 = punit / TB * RUN, vs = pv0 + (e0 >> 2) * 8 + 4 * h + (e0 & 3);
     {
-      if (qcount > (uint32_t)(QC - 256)) {  // room for one unit of the wave
+      if (qcount > (uint32_t)(QC - 64 * RUN)) {  // room for one unit of the wave
         compact();
-        if (qcount > (uint32_t)(QC - 256)) flush();
+        if (qcount > (uint32_t)(QC - 64 * RUN)) flush();
       }
-      bool q[4] = {false, false, false, false};
-      float val[4], ap[4];
+      bool q[RUN], any = false;
+      float val[RUN], ap[RUN];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) val[j] = pend[0][tb][j];
+      for (int j = 0; j < RUN; ++j) q[j] = false;
+#pragma unroll
+      for (int j = 0; j < RUN; ++j) val[j] = pend[0][tb][j];
       if (a.reduce_cast == 1) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = round_bf16(val[j]);
+        for (int j = 0; j < RUN; ++j) val[j] = round_bf16(val[j]);
       } else if (a.reduce_cast == 2) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = round_f16(val[j]);
+        for (int j = 0; j < RUN; ++j) val[j] = round_f16(val[j]);
       }
       const bool row = wb * 32 * TB + tb * 32 + c32 < B;
       if (row && greedy_row[tb]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < RUN; ++j)
           if (vs + j < pvend) sbest[tb] = max_u64(sbest[tb], argmax_key(val[j], (uint32_t)(vs + j)));
       }
       if (row && !greedy_row[tb]) {
-        float x[4];
-        uint32_t idx[4], bits[4];
+        float x[RUN];
+        uint32_t idx[RUN], bits[RUN];
         bool big = false;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < RUN; ++j) {
           x[j] = val[j] * rtp[tb];
           big |= !(fabsf(x[j]) < 1e30f);  // NaN, infinities and the edge of the range: divide
           idx[j] = (uint32_t)(vs + j);
         }
         if (big) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) x[j] = val[j] / tp[tb];
+          for (int j = 0; j < RUN; ++j) x[j] = val[j] / tp[tb];
         }
-        random_bits32_n<4>(key[tb], idx, bits);
+        random_bits32_n<RUN>(key[tb], idx, bits);
         const float am = fmaxf(amax[tb], unord_f32(rowmax[tb * 32]));
         const float thr = am - (2.21e-4f + 1.37e-6f * fminf(fabsf(am), 1e30f));
         float top = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < RUN; ++j) {
           const float t = x[j] + gumbel_fast_from_bits(bits[j]);
           ap[j] = (t != t) ? INFINITY : t;  // NaN only from a NaN logit or temperature
           const bool ok = vs + j < pvend;
@@ -385,9 +463,11 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
         amax[tb] = fmaxf(am, top);
       }
       // queue the marked entries with the whole wave active: slots from a ballot
-      if (__any(q[0] | q[1] | q[2] | q[3])) {
+      #pragma unroll
+      for (int j = 0; j < RUN; ++j) any |= q[j];
+      if (__any(any)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < RUN; ++j) {
           const unsigned long long m = __ballot(q[j]);
           if (q[j]) {
             const uint32_t slot = qcount + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -399,10 +479,10 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
           qcount += (uint32_t)__popcll(m);
         }
       }
-      // shift the row's elements down by four
+      // shift the row's elements down
 #pragma unroll
-      for (int e = 0; e < (S::SMP ? TV : 1) * 16 - 4; ++e)
-        pend[e / 16][tb][e % 16] = pend[(e + 4) / 16][tb][(e + 4) % 16];
+      for (int e = 0; e < (S::SMP ? TV : 1) * 16 - RUN; ++e)
+        pend[e / 16][tb][e % 16] = pend[(e + RUN) / 16][tb][(e + RUN) % 16];
     }
     ++punit;
   };
@@ -496,10 +576,17 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     load_tile_start();
     // as the loop would have left them: X(0) .. X(RX - 2), each W stage RW - RX
     // ahead of the hidden stage issued with it
-    for (int s = 0; s < RW - RX; ++s) issue_w();
-    for (int s = 0; s < RX - 1; ++s) {
-      issue_x();
-      issue_w();
+    if constexpr (NS == 3) {
+      issue_raw();
+      wave_wait<0>();
+      split_raw();
+      for (int s = 0; s < RW - 1; ++s) issue_w();
+    } else {
+      for (int s = 0; s < RW - RX; ++s) issue_w();
+      for (int s = 0; s < RX - 1; ++s) {
+        issue_x();
+        issue_w();
+      }
     }
     for (int t = 0; t < my_tiles; ++t) {
 #pragma unroll
@@ -529,7 +616,7 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     compact();
     flush();
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb) best[tb] = greedy_row[tb] ? sbest[tb] : max_u64(sbest[tb], qbest[tb * 64 + lane]);
+    for (int tb = 0; tb < TB; ++tb) best[tb] = sbest[tb];  // (sampled rows: rowbest)
   } else {
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) best[tb] = bo[tb] ? ((unsigned long long)bo[tb] << 32) | (unsigned long long)(~bi[tb]) : 0ull;
@@ -545,41 +632,49 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     unsigned long long m = kred[0][b];
 #pragma unroll
     for (int q = 1; q < WV; ++q) m = max_u64(m, kred[q][b]);
+    if constexpr (S::SMP) m = max_u64(m, rowbest[b]);
     if (m) (void)after(atomicMax(&a.row_keys[b], m));
   }
   __syncthreads();
   finish_rows(a.row_keys, a.counter, a.B, a.out_ids, a.out_best, (int*)ring);
 }
 
-template <int WT, int MODE, int NBR>
+template <int WT, int MODE, int NBR, int NS>
 static int launch_ring_rows(const LmArgs& a, hipStream_t stream) {
-  using S = RingShape<MODE, NBR>;
+  using S = RingShape<MODE, NBR, NS>;
   const int cus = device_cu_count();
   const int rows = ((a.V + cus - 1) / cus + 7) / 8 * 8;  // every block reads the same share of W, contiguous
-  hipLaunchKernelGGL((lm_head_ring_kernel<WT, MODE, NBR>), dim3((a.V + rows - 1) / rows), dim3(S::NW * 64), 0, stream, a,
-                     rows);
+  hipLaunchKernelGGL((lm_head_ring_kernel<WT, MODE, NBR, NS>), dim3((a.V + rows - 1) / rows), dim3(S::NW * 64), 0, stream,
+                     a, rows);
   NVJSEL_CHECK_LAUNCH("lm_head_ring_kernel");
   return NVJSEL_OK;
 }
 
 template <int WT, int MODE>
 static int launch_ring_mode(const LmArgs& a, hipStream_t stream) {
-  if (a.B <= 32) return launch_ring_rows<WT, MODE, 32>(a, stream);
-  if (a.B <= 64) return launch_ring_rows<WT, MODE, 64>(a, stream);
-  if (a.B <= 128) return launch_ring_rows<WT, MODE, 128>(a, stream);
-  if constexpr (MODE != MODE_SAMPLE) return launch_ring_rows<WT, MODE, 256>(a, stream);
+  if (a.B <= 32) return launch_ring_rows<WT, MODE, 32, 1>(a, stream);
+  if (a.B <= 64) return launch_ring_rows<WT, MODE, 64, 1>(a, stream);
+  if (a.B <= 128) return launch_ring_rows<WT, MODE, 128, 1>(a, stream);
+  if constexpr (MODE != MODE_SAMPLE) return launch_ring_rows<WT, MODE, 256, 1>(a, stream);
   return fail(NVJSEL_EINVAL, "launch_ring: at most 128 sampled rows per pass");
 }
 
-template <int WT>
-static int launch_ring_type(int mode, const LmArgs& a, hipStream_t stream) {
-  if (mode == MODE_GREEDY) return launch_ring_mode<WT, MODE_GREEDY>(a, stream);
-  if (mode == MODE_SAMPLE) return launch_ring_mode<WT, MODE_SAMPLE>(a, stream);
-  return launch_ring_mode<WT, MODE_LOGITS>(a, stream);
+template <int MODE>
+static int launch_ring_f32(const LmArgs& a, hipStream_t stream) {
+  if (a.B <= 32) return launch_ring_rows<DT_BF16, MODE, 32, 3>(a, stream);
+  if (a.B <= 64) return launch_ring_rows<DT_BF16, MODE, 64, 3>(a, stream);
+  return fail(NVJSEL_EINVAL, "launch_ring: at most 64 rows of f32 activations per pass");
 }
 
 int launch_ring(int mode, const LmArgs& a, hipStream_t stream) {
-  return a.weight_dtype == DT_F16 ? launch_ring_type<DT_F16>(mode, a, stream) : launch_ring_type<DT_BF16>(mode, a, stream);
+  auto by_mode = [&](auto fn) -> int {
+    if (mode == MODE_GREEDY) return fn(std::integral_constant<int, MODE_GREEDY>{});
+    if (mode == MODE_SAMPLE) return fn(std::integral_constant<int, MODE_SAMPLE>{});
+    return fn(std::integral_constant<int, MODE_LOGITS>{});
+  };
+  if (a.hidden_dtype == DT_F32) return by_mode([&](auto M) { return launch_ring_f32<decltype(M)::value>(a, stream); });
+  if (a.weight_dtype == DT_F16) return by_mode([&](auto M) { return launch_ring_mode<DT_F16, decltype(M)::value>(a, stream); });
+  return by_mode([&](auto M) { return launch_ring_mode<DT_BF16, decltype(M)::value>(a, stream); });
 }
 
 }  // namespace nvjsel

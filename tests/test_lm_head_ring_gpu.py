@@ -3,7 +3,8 @@ at the edges of its tiles, against the oracle: batch rows around each row
 count it is built for, one to several K stages (H = 64 has one, 192 three:
 fewer and more than the ring's slots), vocabularies of one partial tile, of
 more blocks than rows, and of two tiles per block with a remainder
-(V > 256 x 256), bf16 and f16."""
+(V > 256 x 256), bf16, f16, and f32 activations on bf16 weights (three
+terms per value, 64 rows per pass)."""
 import numpy as np
 import pytest
 import torch
@@ -15,18 +16,19 @@ from tests.gpu_helpers import check_fused_sampled, check_greedy, engine_keys, ke
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(3, 64, 5), (31, 192, 257), (33, 64, 66000), (64, 320, 2055), (65, 128, 66000), (128, 192, 4099),
-          (129, 64, 70001), (256, 192, 1000), (257, 64, 300)]
+          (129, 64, 70001), (256, 192, 1000), (257, 64, 300), (18, 2048, 300)]
 
 
 def _inputs(B, H, V, dt, seed=0):
     rng = np.random.default_rng(B * 1009 + H + V + seed)
     h = torch.from_numpy(rng.standard_normal((B, H)).astype(np.float32)).cuda().to(dt)
-    w = torch.from_numpy((rng.standard_normal((V, H)) * 0.3).astype(np.float32)).cuda().to(dt)
+    w = torch.from_numpy((rng.standard_normal((V, H)) * 0.3).astype(np.float32)).cuda()
+    w = w.to(torch.bfloat16 if dt == torch.float32 else dt)
     z = sel.lm_head_logits(h.float().cpu().numpy(), w.float().cpu().numpy())
-    return rng, h, w, z, (1 if dt == torch.bfloat16 else 2)
+    return rng, h, w, z, {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dt]
 
 
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,H,V", SHAPES)
 def test_greedy_and_logits(B, H, V, dt):
     _, h, w, z, rc = _inputs(B, H, V, dt)
@@ -36,17 +38,17 @@ def test_greedy_and_logits(B, H, V, dt):
     check_greedy(ids.cpu().numpy(), z, rc, f"ring greedy {dt} {B} {H} {V}")
     got = logits.float().cpu().numpy().astype(np.float64)
     # fp32 sums of H products (H 2^-24 sum |h w| <= H 2^-24 |h| |w|) and one
-    # rounding to the 16-bit type (half an ulp: 2^-9 bf16, 2^-12 f16)
+    # rounding to the 16-bit type (within an ulp: 2^-8 bf16, 2^-11 f16, f32 as summed)
     hn = np.linalg.norm(h.float().cpu().numpy(), axis=1)[:, None]
     wn = np.linalg.norm(w.float().cpu().numpy(), axis=1)[None, :]
-    tol = H * 2.0 ** -24 * hn * wn * 2 + np.abs(z) * (2.0 ** -8 if rc == 1 else 2.0 ** -11) + 1e-7
+    tol = H * 2.0 ** -24 * hn * wn * 2 + np.abs(z) * {0: 2.0 ** -24, 1: 2.0 ** -8, 2: 2.0 ** -11}[rc] + 1e-7
     assert (np.abs(got - z) <= tol).all()
     # the winning logit is the row's largest stored logit, at its first index
     np.testing.assert_array_equal(best.cpu().numpy(), logits.float().max(dim=1).values.cpu().numpy())
     np.testing.assert_array_equal(ids.cpu().numpy().reshape(-1), got.argmax(axis=1))
 
 
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,H,V", [s for s in SHAPES if s[0] <= 128 or s[0] == 257])
 def test_sample(B, H, V, dt):
     rng, h, w, z, rc = _inputs(B, H, V, dt, 1)
