@@ -596,11 +596,11 @@ __device__ __forceinline__ unsigned long long wave_gumbel(const SampleArgs& a, i
 
 // ------------------------------------------------------------------ top-k rows from candidates
 // A FILTER row with k <= 256: the row floor is the larger of the largest chunk
-// floor and the k-th largest lane maximum the scan published (four per wave);
+// floor and the k-th largest lane maximum the scan published (tops_shift);
 // the candidates at or above it (about k of them) are rank-sorted in LDS, and
 // top-k, top-p and the exact Gumbel-max read the sorted prefix.
 static constexpr int kTops = 8;        // lane maxima ranked per wave (tier A bound)
-static constexpr int kTopsPub = 4;     // of them published per wave (row floor)
+static constexpr int kTopsPub = 8;     // most of them published per wave (row floor)
 static constexpr int kTopsChunks = 64; // chunks whose tops bound the row floor (<= 1024 values)
 static constexpr int kFinCap = 512;    // survivors sorted in LDS
 
@@ -615,6 +615,22 @@ struct FinishShared {
   uint32_t hist[256];
   uint32_t n, kf, tau, rem, nk;
 };
+
+// log2 of the lane maximums published per wave: eight on fewer than 16 chunks,
+// where four may not reach well past k, else four (V = 50,257, k = 100 at 7
+// chunks 197 -> 33 us; at 16 chunks reading eight slowed a mixed call of 256
+// rows by 1%).
+__device__ __forceinline__ int tops_shift(const SampleArgs& a) { return a.nchunks < 16 ? 3 : 2; }
+
+// Whether the scan writes a top-k row's tier B too: always for nvjsel_topk; for
+// the sampler where the row's chunks hold so few of the k that some chunk's
+// tier A (at least 32 elements) may end above the row floor, which is the k-th
+// of the lane maximums the chunks publish (k = 100 below 7 chunks).  A row
+// whose lists stop short takes a whole-row descent: V = 37,888, 67 rows, k =
+// 100 152 us against 26-39.
+__device__ __forceinline__ bool scan_tier_b(const SampleArgs& a, const RowParams& rp) {
+  return a.topk > 0 || ((kThreads / 64) * a.nchunks << tops_shift(a)) < 2 * rp.k;
+}
 
 // The first loads of a fast top-k row, issued by select before it reduces the
 // chunk maxima so that both are in flight together: each chunk's tier A count
@@ -640,12 +656,13 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPr
     pf.fl_a = a.cand_floor_a[i];
     pf.fl = a.cand_floor[i];
   }
-  const int nvals = min(NC, kTopsChunks) * (kThreads / 64) * kTopsPub;
+  const int ts = tops_shift(a);
+  const int nvals = (min(NC, kTopsChunks) * (kThreads / 64)) << ts;
   const float* tops = a.lane_tops + (size_t)b * NC * (kThreads / 64) * kTopsPub;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = (int)threadIdx.x + kThreads * i;
-    pf.key[i] = j < nvals ? radix_key(tops[j]) >> 16 : 0u;
+    pf.key[i] = j < nvals ? radix_key(tops[(j >> ts) * kTopsPub + (j & ((1 << ts) - 1))]) >> 16 : 0u;
   }
   // the first list entries the gather reads, requested now rather than once
   // the row floor is known (inside each chunk's list area; entries past the
@@ -691,7 +708,7 @@ __device__ __forceinline__ uint32_t row_tops_kth(const uint32_t (&key)[4], int k
 // lane maximum, largest chunk floor) <= the row's k-th largest, so the row's
 // top-k (ties included) is a prefix.  Returns -1 when a chunk's list
 // overflowed, F falls below a chunk's tier A and the list holds no tier B
-// (the sampler's), or the survivors do not fit in LDS.
+// (scan_tier_b), or the survivors do not fit in LDS.
 __device__ int topk_sorted_survivors(const SampleArgs& a, int b, const RowParams& rp, const TopkPrefetch& pf,
                                      FinishShared& s) {
   const int NC = a.nchunks, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -717,7 +734,7 @@ __device__ int topk_sorted_survivors(const SampleArgs& a, int b, const RowParams
         need = (int)s.cnt_a[c];
       } else {
         need = (int)s.cnt[c];
-        bad |= a.topk == 0;  // the sampler's lists stop at tier A
+        bad |= !scan_tier_b(a, rp);  // the list stops at tier A
       }
       bad |= need > kCandCap;
       need = min(need, kCandCap);
@@ -1053,13 +1070,13 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     // the lane maxima as radix keys (lanes holding no element of the row: 0,
     // below every value), sorted: lane t holds the t-th largest.  The
     // kk-th largest gives the wave floor (its top 16 bits: the largest
-    // prefix that kk lane maxima reach), lanes 0..kTopsPub-1 publish the
+    // prefix that kk lane maxima reach), the first lanes publish the
     // largest lane maxima, lane kTops-1 the kTops-th (-inf fills)
     const uint32_t sk = wave_sort_desc(r.vok[0] ? radix_key(tv) : 0u);
     wfloor = kk ? ((uint32_t)__builtin_amdgcn_readlane((int)sk, (int)kk - 1) >> 16) << 16 : 0xFFFFFFFFu;
     const float sv = sk > 0x007FFFFFu ? radix_value(sk) : -INFINITY;
     float* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
-    if (lane < kTopsPub) tops[lane] = sv;
+    if (lane < 1 << tops_shift(a)) tops[lane] = sv;
     if (lane == kTops - 1) sh.wtop[wave] = sv;
   } else if (topk && lane < kTopsPub) {
     if (lane == 0) sh.wtop[wave] = -INFINITY;
@@ -1122,14 +1139,15 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
   const float theta_v = theta > 0x007FFFFFu ? radix_value(theta) : -INFINITY;
   // Tier A, written first: candidates at or above t_a = min over waves of the
   // wave's kTops-th largest lane maximum (the chunk holds at least
-  // 4 * kTops elements >= t_a).  A row floor >= t_a needs only tier A, and the
-  // sampler's fast path takes no other (the rare row that needs more takes
-  // the exact path), so only nvjsel_topk writes tier B: the rest down to theta.
+  // 4 * kTops elements >= t_a).  A row floor >= t_a needs only tier A; tier B,
+  // the rest down to theta, is written where the floor may lie lower
+  // (scan_tier_b; elsewhere the rare row that needs it takes the exact path).
   float t_a = sh.wtop[0];
 #pragma unroll
   for (int w = 1; w < kThreads / 64; ++w) t_a = fminf(t_a, sh.wtop[w]);
   const float th_a = fmaxf(t_a, theta_v);
-  const float lo = a.topk > 0 ? theta_v : th_a;
+  const bool tier_b = scan_tier_b(a, rp);  // block-uniform
+  const float lo = tier_b ? theta_v : th_a;
   // vectors holding a candidate, walked sparsely: each lane visits only its own
   uint32_t pend = 0;
   if (!nan_chunk) {
@@ -1167,7 +1185,7 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
   if (lane == 0 && (wtot & 0xFFFFu)) wbase = atomicAdd(&sh.cnt, wtot & 0xFFFFu);
   uint32_t slot_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)wbase) + ((incl - mine) & 0xFFFFu);
   uint32_t slot_b = 0;
-  if (a.topk > 0) {
+  if (tier_b) {
     lds_barrier();
     const uint32_t n_a = sh.cnt;
     wbase = 0;
