@@ -674,8 +674,8 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
   const int ew = wave - GW;                      // epilogue wave index
   const int el = (ew < 0 ? 0 : ew) * 64 + lane;  // epilogue lane id
   const int erow = el % ROWS, evq = el / ROWS;   // batch row, vocab run (EPL rows)
-  float tp = 1.0f;
-  bool greedy_row = true, unit_tp = true;
+  float tp = 1.0f, rtp = 1.0f;
+  bool greedy_row = true;
   TfKey key = tf_key(0u, 0u);
   unsigned long long best = 0;
   float amax = -INFINITY;
@@ -693,7 +693,7 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
     __builtin_amdgcn_sched_barrier(0);
   };
   // exact scores of the queued elements, a full wave at a time; an entry holds
-  // x and (vocab << 6 | lane that found it); results fold into qbest[lane]
+  // the logit and (vocab << 6 | lane that found it); results fold into qbest[lane]
   auto flush = [&]() {
     if constexpr (MODE == MODE_SAMPLE) {
       const uint32_t n = qcount;
@@ -705,7 +705,8 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
         // the shuffles run with the whole wave active
         const TfKey k2{(uint32_t)__shfl((int)key.k0, (int)src, 64), (uint32_t)__shfl((int)key.k1, (int)src, 64),
                        (uint32_t)__shfl((int)key.k2, (int)src, 64)};
-        if (live) atomicMax(&qbest[ew][src], argmax_key(qx[ew][e] + gumbel_at(k2, v), v));
+        const float t2 = __shfl(tp, (int)src, 64);
+        if (live) atomicMax(&qbest[ew][src], argmax_key(qx[ew][e] / t2 + gumbel_at(k2, v), v));
       }
       qcount = 0;
     }
@@ -726,8 +727,7 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
         const float ap = live ? qa[ew][e] : -INFINITY;
         const uint32_t pv = live ? qv[ew][e] : 0u;
         const float am = __shfl(amax, (int)(pv & 63u), 64);
-        const float slack = 2e-4f + 4.8e-7f * (fminf(fabsf(ap), 1e30f) + fminf(fabsf(am), 1e30f));
-        const bool keep = live && !(ap + slack < am);
+        const bool keep = live && !(ap + score_slack(ap, am) < am);
         const unsigned long long m = __ballot(keep);
         if (keep) {
           const uint32_t slot = nk + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -801,7 +801,7 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
       const float t = erow < B ? a.temperature[erow] : 0.0f;
       greedy_row = (t <= 0.0f);
       tp = temp_floor(t);
-      unit_tp = (tp == 1.0f);  // x / 1 == x exactly
+      rtp = 1.0f / tp;
       if (erow < B) key = tf_key(a.keys[2 * erow], a.keys[2 * erow + 1]);
       qbest[ew][lane] = 0;
     }
@@ -907,7 +907,7 @@ __global__ void __launch_bounds__((GW + NB * EPM) * 64) lm_head_tile_kernel(LmAr
           for (int e = 0; e < EPL; ++e)
             if (v0 + e < V) store_logit(a, erow, v0 + e, apply_cast(raw[e], a.reduce_cast));
         } else {
-          score_run<MODE, EPL>(raw, v0, V, a.reduce_cast, greedy_row, unit_tp, tp, key, amax, best, q, xq, aq);
+          score_run<MODE, EPL>(raw, v0, V, a.reduce_cast, greedy_row, rtp, tp, key, amax, best, q, xq, aq);
         }
       }
       if constexpr (MODE == MODE_SAMPLE) {

@@ -185,16 +185,23 @@ __device__ __forceinline__ void finish_rows(unsigned long long* row_keys, unsign
 // Scores N consecutive vocabulary entries v0.. of one batch row (raw fp32
 // dots).  Greedy: folds argmax keys into `best`.  Sample: computes the fast
 // approximate scores for all N in one straight-line block (N interleaved
-// Threefry chains) and marks in q[] (scaled logit xq[], approximate score aq[])
-// every entry that can still be the row's exact maximum:
-// |approx - exact| <= d(s) = 1e-4 + 4.8e-7 |s| (hardware log error ~1e-6 on the
-// draw, plus one ulp of the sum), so the exact maximum j has
+// Threefry chains) and marks in q[] (logit xq[], approximate score aq[]) every
+// entry that can still be the row's exact maximum.  The approximate score
+// multiplies with rtp = 1 / tp (the exact rescoring divides; a division per
+// draw cost ~10% of the draws' time).  |approx - exact| <= d(s) = 1e-4 + 4.8e-7
+// |s| + 1.8e-7 |x|, |x| <= |s| + 16 (hardware log error ~1e-6 on the draw, one
+// ulp of the sum, three roundings of the product), so the exact maximum j has
 // approx_j >= approx_k - d(s_j) - d(s_k) for every k and is queued when it
-// arrives, whatever set of approximate scores `amax` is the maximum of.
-// Magnitudes are clamped so -inf stays -inf; a NaN scaled logit scores +inf.
+// arrives, whatever set of approximate scores `amax` is the maximum of
+// (score_slack: the two together).  Magnitudes are clamped so -inf stays -inf;
+// a NaN scaled logit scores +inf.
+__device__ __forceinline__ float score_slack(float ap, float am) {
+  return 2.2e-4f + 6.8e-7f * (fminf(fabsf(ap), 1e30f) + fminf(fabsf(am), 1e30f));
+}
+
 template <int MODE, int N>
 __device__ __forceinline__ void score_run(const float (&raw)[N], int v0, int V, int reduce_cast, bool greedy_row,
-                                          bool unit_tp, float tp, const TfKey& key, float& amax,
+                                          float rtp, float tp, const TfKey& key, float& amax,
                                           unsigned long long& best, bool (&q)[N], float (&xq)[N], float (&aq)[N]) {
   // one branch per run, not per element: the cast and the bounds are uniform
   float val[N];
@@ -212,8 +219,11 @@ __device__ __forceinline__ void score_run(const float (&raw)[N], int v0, int V, 
     float xv[N], ap[N];
     uint32_t bits[N];
 #pragma unroll
-    for (int e = 0; e < N; ++e) xv[e] = val[e];
-    if (!unit_tp) {
+    for (int e = 0; e < N; ++e) xv[e] = val[e] * rtp;
+    float mag = fabsf(xv[0]);
+#pragma unroll
+    for (int e = 1; e < N; ++e) mag = fmaxf(mag, fabsf(xv[e]));
+    if (!(mag < 1e30f)) {  // infinities and the edge of the float range: divide
 #pragma unroll
       for (int e = 0; e < N; ++e) xv[e] = val[e] / tp;
     }
@@ -230,18 +240,18 @@ __device__ __forceinline__ void score_run(const float (&raw)[N], int v0, int V, 
     }
     // every draw feeds an unconditional select, so none is sunk into a branch.
     // One threshold per run instead of the per-entry slack: an entry that
-    // passes ap + 2e-4 + 4.8e-7 (|ap| + |am|) >= am has |ap| <= |am| + slack,
-    // so slack <= 2.01e-4 + 9.61e-7 |am| and ap >= am - that bound: the
-    // queued set only grows (the filter before exact rescoring applies the
-    // per-entry test).  am = -inf queues every entry, am = +inf only +inf.
+    // passes ap + score_slack(ap, am) >= am has |ap| <= |am| + slack, so slack
+    // <= 2.21e-4 + 1.37e-6 |am| and ap >= am - that bound: the queued set only
+    // grows (the filter before exact rescoring applies the per-entry test).
+    // am = -inf queues every entry, am = +inf only +inf.
     const float am = amax;
-    const float thr = am - (2.01e-4f + 9.61e-7f * fminf(fabsf(am), 1e30f));
+    const float thr = am - (2.21e-4f + 1.37e-6f * fminf(fabsf(am), 1e30f));
     const bool all_in = v0 + N <= V;  // uniform per run except in the last tile
 #pragma unroll
     for (int e = 0; e < N; ++e) {
       const bool ok = all_in || v0 + e < V;
       q[e] = ok && ap[e] >= thr;
-      xq[e] = xv[e];
+      xq[e] = val[e];
       aq[e] = ap[e];
       amax = fmaxf(amax, ok ? ap[e] : -INFINITY);
     }

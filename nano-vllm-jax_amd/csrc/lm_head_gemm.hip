@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
   __shared__ u32x4_t Bs[2][NS][Q * XB];
   __shared__ unsigned long long kred[VH][KBR];
   // sample mode: per-wave queue of entries that may be their row's maximum
-  // (scaled logit, approximate score, vocab << 7 | tb << 6 | lane) and the
+  // (logit, approximate score, vocab << 7 | tb << 6 | lane) and the
   // exact best key of each (lane, tb) row slot
   constexpr bool SMP = MODE == MODE_SAMPLE;
   constexpr int NW = NT / 64;
@@ -318,8 +318,8 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
   };
   uint32_t bo[2] = {0u, 0u}, bi[2] = {0u, 0u};  // running best: ordered value, row
   // sample mode: the lane's two batch rows bj * 64 + tb * 32 + c32
-  float tp[2] = {1.0f, 1.0f}, amax[2] = {-INFINITY, -INFINITY};
-  bool greedy_row[2] = {true, true}, unit_tp[2] = {true, true};
+  float tp[2] = {1.0f, 1.0f}, rtp[2] = {1.0f, 1.0f}, amax[2] = {-INFINITY, -INFINITY};
+  bool greedy_row[2] = {true, true};
   TfKey key[2] = {tf_key(0u, 0u), tf_key(0u, 0u)};
   unsigned long long sbest[2] = {0ull, 0ull};
   uint32_t qcount = 0;  // wave-uniform
@@ -330,7 +330,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
       const float t = b < B ? a.temperature[b] : 0.0f;
       greedy_row[tb] = (t <= 0.0f);
       tp[tb] = temp_floor(t);
-      unit_tp[tb] = (tp[tb] == 1.0f);  // x / 1 == x exactly
+      rtp[tb] = 1.0f / tp[tb];
       if (b < B) key[tb] = tf_key(a.keys[2 * b], a.keys[2 * b + 1]);
       gqbest[wave][tb * 64 + lane] = 0ull;
     }
@@ -350,8 +350,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
       const int sl = (int)(pv & 63u);
       const float a0 = __shfl(amax[0], sl, 64), a1 = __shfl(amax[1], sl, 64);
       const float am = (pv & 64u) ? a1 : a0;
-      const float slack = 2e-4f + 4.8e-7f * (fminf(fabsf(ap), 1e30f) + fminf(fabsf(am), 1e30f));
-      const bool keep = live && !(ap + slack < am);
+      const bool keep = live && !(ap + score_slack(ap, am) < am);
       const unsigned long long m = __ballot(keep);
       if (keep) {
         const uint32_t slot = nk + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -383,7 +382,8 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
       }
       const TfKey k2{t1 ? kw[1][0] : kw[0][0], t1 ? kw[1][1] : kw[0][1], t1 ? kw[1][2] : kw[0][2]};
       const uint32_t v = pv >> 7;
-      if (live) atomicMax(&gqbest[wave][pv & 127u], argmax_key(gqx[wave][e] + gumbel_at(k2, v), v));
+      const float u0 = __shfl(tp[0], sl, 64), u1 = __shfl(tp[1], sl, 64);
+      if (live) atomicMax(&gqbest[wave][pv & 127u], argmax_key(gqx[wave][e] / (t1 ? u1 : u0) + gumbel_at(k2, v), v));
     }
     qcount = 0;
   };
@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
           float xq[2], aq[2];
           if (b < B) {
             const float raw[2] = {acc[0][tb][2 * qq], acc[0][tb][2 * qq + 1]};
-            score_run<MODE_SAMPLE, 2>(raw, vs, V, a.reduce_cast, greedy_row[tb], unit_tp[tb], tp[tb], key[tb],
+            score_run<MODE_SAMPLE, 2>(raw, vs, V, a.reduce_cast, greedy_row[tb], rtp[tb], tp[tb], key[tb],
                                       amax[tb], sbest[tb], q, xq, aq);
           }
           // queue the marked entries with the whole wave active: slots from a ballot

@@ -331,13 +331,6 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
       rowmax[tb * 32] = 0u;
     }
   }
-  // Bound on |approximate - exact| of two scores ap, am together: 1e-4 covers
-  // the hardware log's error on a draw (1.91e-6) with room, 4.8e-7 |s| the
-  // rounding of the sum, 1.8e-7 |x| (|x| <= |s| + 16) the product with 1 / T'
-  // in place of the division.  Magnitudes are clamped so -inf stays -inf.
-  auto slack = [](float ap, float am) NVJSEL_INLINE {
-    return 2.2e-4f + 6.8e-7f * (fminf(fabsf(ap), 1e30f) + fminf(fabsf(am), 1e30f));
-  };
   // drops queued entries that can no longer be their row's maximum (the test
   // each passed when queued, against a maximum that has only grown since);
   // compaction in place, a 64-entry group read before any survivor is written
@@ -356,7 +349,7 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
         const float a1 = __shfl(amax[1], sl, 64);
         if (pv & 64u) am = a1;
       }
-      const bool keep = live && !(ap + slack(ap, am) < am);
+      const bool keep = live && !(ap + score_slack(ap, am) < am);
       const unsigned long long m = __ballot(keep);
       if (keep) {
         const uint32_t slot = nk + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
