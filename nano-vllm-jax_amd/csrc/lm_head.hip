@@ -1332,7 +1332,7 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // activations of one type).  Greedy and logits above the GEMV's rows: H =
   // 1024, V = 248k, B = 16 / 64 / 100 / 256 76 / 78 / 88 / 136 us against 78 /
   // 81 / 158 / 177 in 64-row tile passes and the blocked GEMM; logits B = 64 /
-  // 80 / 256 102 / 118 / 206 against 149 / 240 / 273; H = 2560, V = 152k, B =
+  // 80 / 256 99 / 114 / 184 against 149 / 240 / 273; H = 2560, V = 152k, B =
   // 16 / 64 120 / 134 against 259 / 1010 in the straight-to-registers kernel.
   // With the norm in the call (a prologue and a zeroing launch, ~11 us) the
   // tile kernel's fused prologue stays up to 32 rows (85-88 us; 64 rows 100

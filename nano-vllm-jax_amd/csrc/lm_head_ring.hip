@@ -23,8 +23,9 @@
 //    the index looked up by comparing raw values with the smallest float that
 //    rounds to that maximum (a lookup per 32 x 32 tile with rounded values:
 //    B = 128 / 256 106 / 162 us against 93 / 147).
-//  * Logits: operands swapped, so that 32 lanes store 64 contiguous bytes of
-//    one row (B = 80 240 -> 118 us).
+//  * Logits: operands swapped, so that 32 lanes hold 64 contiguous bytes of
+//    one row, and quads of lanes transposed for 8-byte stores (B = 80 / 256
+//    2-byte stores 118 / 206 us, 8-byte 114 / 184; 32-byte runs 240 / 273).
 //  * Sampling: a finished tile's logits stay in registers and are scored in
 //    small units beside the next tile's stages (B = 64 136 -> 117-123 us, B =
 //    128 224 -> 183); the waves share the rows' maxima through the LDS, so few
@@ -124,6 +125,31 @@ __device__ __forceinline__ uint2 next_term(float (&v)[4]) {
 template <int N>
 __device__ __forceinline__ void wave_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// x[j]: this lane's value of row j, its column the lane's place in its quad.
+// Lane j of the quad gets row j's four columns as 16-bit values (bf16 or f16,
+// round to nearest even).
+__device__ __forceinline__ uint2 quad_transpose16(const float (&x)[4], int dtype, int lane) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  uint32_t r02, r13;  // rows 0 | 2 << 16 and 1 | 3 << 16 of this column
+  if (dtype == DT_BF16) {
+    r02 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[0], x[2]}), bf16x2_t));
+    r13 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[1], x[3]}), bf16x2_t));
+  } else {
+    r02 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[0], x[2]}), f16x2));
+    r13 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[1], x[3]}), f16x2));
+  }
+  const bool odd = lane & 1, high = lane & 2;
+  // with lane ^ 1: an even lane keeps rows 0 and 2, an odd one rows 1 and 3
+  const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(odd ? r02 : r13), 0xB1, 0xF, 0xF, false);
+  const uint32_t own = odd ? r13 : r02, lo = odd ? got : own, hi = odd ? own : got;
+  const uint32_t p = __builtin_amdgcn_perm(hi, lo, 0x05040100u);  // row (odd): this column pair
+  const uint32_t q = __builtin_amdgcn_perm(hi, lo, 0x07060302u);  // row 2 + (odd)
+  // with lane ^ 2: the low pair keeps rows 0 and 1, the high pair rows 2 and 3
+  const uint32_t g2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(high ? p : q), 0x4E, 0xF, 0xF, false);
+  return high ? uint2{g2, q} : uint2{p, g2};
 }
 
 // rows: vocabulary rows per block (a multiple of 8).
@@ -491,16 +517,30 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     const int v0 = t0 + wv * TV * 32;
     if constexpr (MODE == MODE_LOGITS) {
       // operands swapped: D[batch 8 (e >> 2) + 4 h + (e & 3)][vocab c32], so
-      // 32 lanes store 32 consecutive logits of one row
+      // 32 lanes hold 32 consecutive logits of one row.  16-bit logits at
+      // addresses that allow it are transposed in quads of lanes (four rows x
+      // four columns) and stored 8 bytes per lane.
+      const bool quads = a.out_dtype != DT_F32 && ((a.V | (int)a.out_stride) & 3) == 0 && (((uintptr_t)a.out_logits) & 7) == 0;
 #pragma unroll
       for (int tv = 0; tv < TV; ++tv) {
         const int v = v0 + tv * 32 + c32;
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int b = wb * 32 * TB + tb * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-            if (v < vend && b < B) store_logit(a, b, v, apply_cast(acc[tv][tb][e], a.reduce_cast));
+          for (int i = 0; i < 4; ++i) {
+            const int b = wb * 32 * TB + tb * 32 + 8 * i + 4 * h;
+            float x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = apply_cast(acc[tv][tb][4 * i + j], a.reduce_cast);
+            if (quads) {
+              const uint2 q = quad_transpose16(x, a.out_dtype, lane);
+              if (v < vend && b + (lane & 3) < B)  // (vend is a multiple of 4: whole quads)
+                *(uint2*)((uint16_t*)a.out_logits + (size_t)(b + (lane & 3)) * (size_t)a.out_stride + (v & ~3)) = q;
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                if (v < vend && b + j < B) store_logit(a, b + j, v, x[j]);
+            }
           }
       }
     } else if constexpr (S::SMP) {

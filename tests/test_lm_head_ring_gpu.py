@@ -87,25 +87,28 @@ def test_ties_nan_and_infinities(reduce_cast):
     assert ids[1] == 777
 
 
-def test_sample_extreme_temperatures_and_nan():
+@pytest.mark.parametrize("B,H,layout", [(80, 64, "vh"), (40, 1024, "vh"), (20, 64, "hv"), (140, 64, "vh")])
+def test_sample_extreme_temperatures_and_nan(B, H, layout):
     """Tiny and huge temperatures (products with 1 / T' out of the float range
-    are divided instead), a NaN temperature and a NaN logit row."""
-    B, H, V = 80, 64, 3001
+    are divided instead), a NaN temperature and a NaN logit row, in every
+    kernel that scores with the product."""
+    V = 3001
     rng = np.random.default_rng(9)
     h = rng.standard_normal((B, H)).astype(np.float32)
     w = (rng.standard_normal((V, H)) * 0.3).astype(np.float32)
     hb = torch.from_numpy(h).cuda().to(torch.bfloat16)
     wb = torch.from_numpy(w).cuda().to(torch.bfloat16)
+    wo = wb if layout == "vh" else wb.T.contiguous()
     T = [float(x) for x in rng.choice([1e-7, 1e-3, 0.5, 50.0, 1e30], B)]
     keys = engine_keys(B, 3)
-    ids = nvjsel.lm_head_sample_token_ids(hb, wb, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
-                                          weight_layout="vh").cpu().numpy()
+    ids = nvjsel.lm_head_sample_token_ids(hb, wo, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                          weight_layout=layout).cpu().numpy()
     z = sel.lm_head_logits(hb.float().cpu().numpy(), wb.float().cpu().numpy())
     check_fused_sampled(ids, z, T, keys, 1, "ring sample extreme T")
     hb[4, 0] = float("nan")
     T[9] = float("nan")
-    ids = nvjsel.lm_head_sample_token_ids(hb, wb, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
-                                          weight_layout="vh").cpu().numpy()
+    ids = nvjsel.lm_head_sample_token_ids(hb, wo, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                          weight_layout=layout).cpu().numpy()
     assert ids[4] == 0 and ids[9] == 0  # every score a NaN: the first
     ok = [b for b in range(B) if b not in (4, 9)]
     check_fused_sampled(ids[ok], z[ok], [T[b] for b in ok], keys[ok], 1, "ring sample beside NaN rows")
