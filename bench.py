@@ -346,7 +346,7 @@ def build_configs(torch, which, with_cpu):
                 "x4": "greedy LM-head top-1, B=8, W [1024,248320] bf16 ([H,V])",
                 "x5": "greedy LM-head top-1, B=8, fp32 activations x W [248320,1024] bf16 (one W pass)",
                 "x6": "greedy LM-head top-1, B=256, bf16 x W [248320,1024] bf16 (one W pass, blocked GEMM)"}[name]
-        kern = {"x5": "lm_head_tile_kernel", "x6": "lm_head_gemm_kernel"}.get(name, "lm_head_hv_kernel")
+        kern = {"x5": "lm_head_tile_kernel", "x6": "lm_head_ring_kernel"}.get(name, "lm_head_hv_kernel")
         tag = "hv" if layout else {"x5": "f32act", "x6": "gemm"}[name]
         cfgs.append(Cfg(f"{name}_{tag}_greedy_b{B}", B,
                         V_FULL * H_FULL * 2 + B * H_FULL * h.element_size(), launch, 2, kern, desc))
