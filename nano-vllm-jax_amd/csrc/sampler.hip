@@ -616,11 +616,11 @@ struct FinishShared {
   uint32_t n, kf, tau, rem, nk;
 };
 
-// log2 of the lane maximums published per wave: eight on fewer than 16 chunks,
-// where four may not reach well past k, else four (V = 50,257, k = 100 at 7
-// chunks 197 -> 33 us; at 16 chunks reading eight slowed a mixed call of 256
-// rows by 1%).
-__device__ __forceinline__ int tops_shift(const SampleArgs& a) { return a.nchunks < 16 ? 3 : 2; }
+// log2 of the lane maximums published per wave: eight on fewer than 13 chunks,
+// where four per wave are fewer than twice a k of 100, else four (V = 50,257, k
+// = 100 at 7 chunks 197 -> 33 us; reading eight slowed mixed calls at 14 and
+// 16 chunks by 0.6-1%).
+__device__ __forceinline__ int tops_shift(const SampleArgs& a) { return a.nchunks < 13 ? 3 : 2; }
 
 // Whether the scan writes a top-k row's tier B too: always for nvjsel_topk; for
 // the sampler where the row's chunks hold so few of the k that some chunk's
