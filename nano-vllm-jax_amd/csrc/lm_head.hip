@@ -1387,8 +1387,10 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // value, from 9 rows; at 65-128 rows passes of 64 rows through its narrow
   // layout while more than 8 rows are left, then a streaming pass (greedy B =
   // 65 / 72 / 96-128 ~262 / ~278 / ~350 us, sampled ~302 / ~333 / ~409-434 us,
-  // against ~376-396 / ~494-504 us in the 256-row kernel)
-  const bool mix3 = gemm_ok && hv_gemm_ok && eff_dtype == NVJSEL_F32 && batch > 64 && batch <= kMix3MaxBatch;
+  // against ~376-396 / ~494-504 us in the 256-row kernel); where the streaming
+  // kernel's LDS does not fit (8 rows from H = 5120) the 256-row kernel takes
+  // the whole call
+  const bool mix3 = gemm_ok && hv_gemm_ok && hv && eff_dtype == NVJSEL_F32 && batch > 64 && batch <= kMix3MaxBatch;
   const int mix_rest = mode == MODE_SAMPLE ? kGemm3HvMinBatchSample : kGemm3HvMinBatch;
   const bool gemm3 = !mix3 && gemm_ok && hv_gemm_ok && eff_dtype == NVJSEL_F32 && batch > mix_rest;
   const bool fused_prenorm = prenorm && !gemm && !gemm3 && !mix3 &&
@@ -1428,6 +1430,7 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
                      : mix3 ? (g3 ? 64 : chunk)
                             : (chunk > 0 ? chunk : batch);
     nb = left < step ? left : step;
+    if (nb <= 0) return fail(NVJSEL_EINVAL, "lm_head: a pass of no rows");  // (every pass above takes some)
     a.W = weight;
     a.hidden = (const char*)hidden + (size_t)b0 * H * dtype_size(hidden_dtype);
     a.hidden_dtype = hidden_dtype;

@@ -67,3 +67,20 @@ def test_winner_in_the_last_partial_group(B, col):
     w[H - 1, col] = 2.0
     ids, best = nvjsel.lm_head_greedy_top1_hip(h, w, weight_layout="hv", return_best=True)
     assert (ids.cpu().numpy() == col).all() and (best.cpu().numpy() == 2.0).all()
+
+
+@pytest.mark.parametrize("B", [65, 66, 72, 73, 128])
+@pytest.mark.parametrize("V", [136, 129])
+def test_f32_rows_past_the_streaming_kernels_lds(V, B):
+    """H = 5120: eight streaming rows do not fit the LDS, so 65-128 f32 rows
+    have no streaming pass to end on and one GEMM pass takes them all."""
+    H = 5120
+    _, h, w, z, rc = _case(B, H, V, torch.float32, torch.bfloat16, 2)
+    ids = nvjsel.lm_head_greedy_top1_hip(h, w, weight_layout="hv")
+    logits = nvjsel.lm_head_logits_hip(h, w, weight_layout="hv")
+    torch.cuda.synchronize()
+    check_greedy(ids.cpu().numpy(), z, rc, f"hv f32 B={B} H={H} V={V}")
+    # fp32 sums of three products per element: 3 H 2^-24 sum |h w| at most, sum |h w| <= |h| |w|
+    hn = np.linalg.norm(h.float().cpu().numpy(), axis=1)[:, None]
+    wn = np.linalg.norm(w.float().cpu().numpy(), axis=0)[None, :]
+    assert (np.abs(logits.cpu().numpy().astype(np.float64) - z) <= 3 * H * 2.0 ** -24 * hn * wn).all()
