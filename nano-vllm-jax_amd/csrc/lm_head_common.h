@@ -284,6 +284,77 @@ __device__ __forceinline__ void split_terms(const float (&v)[8], u32x4_t (&hb)[N
   }
 }
 
+// NaN logits of f32 hidden in three bf16 terms, summed again from the f32
+// values.  The split holds for finite operands: an infinite value (or one that
+// rounds to bf16's infinity) leaves NaN remainders, and an infinite weight
+// meets lower terms that are zero or of the other sign, where the fp32
+// products have an infinity, or a finite sum.  Rows that hold a NaN keep it.
+// d: the wave's 32 x 32 tiles; at(tv, e, b, v): batch and vocabulary row of
+// element e of tile (tv, TBI) of this lane, whether it is a live one; ROWLANE: a lane's elements all belong to one batch row.  The whole
+// wave sums each such logit (V = 248,320, H = 1024, 64 [V, H] / 24 [H, V] rows,
+// one of them holding an infinity: 2.5 ms in place of 117 / 198 us; a NaN:
+// 137 / 213 us); finite operands pay the callers' test for a NaN, out of a
+// maximum over the tile's values (within the runs' noise).
+__device__ __forceinline__ bool row_has_nan(const LmArgs& a, int b, int lane) {
+  const float* x = (const float*)a.hidden + (size_t)b * a.H;
+  bool nan = false;
+  for (int k = lane; k < a.H; k += 64) nan |= x[k] != x[k];
+  return __any(nan);
+}
+__device__ __forceinline__ float wave_dot_f32(const LmArgs& a, int b, int v, int lane) {
+  const float* x = (const float*)a.hidden + (size_t)b * a.H;
+  const uint16_t* w = (const uint16_t*)a.W + (a.layout == NVJSEL_W_VH ? (size_t)v * a.H : (size_t)v);
+  const size_t step = a.layout == NVJSEL_W_VH ? 1 : (size_t)a.V;
+  float s = 0.0f;
+  for (int k = lane; k < a.H; k += 64) s = fmaf(x[k], __uint_as_float((uint32_t)w[k * step] << 16), s);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  return s;
+}
+template <int TBI, bool ROWLANE, int TV, int TB, typename At>
+__device__ __forceinline__ void redo_nan_logits(const LmArgs& a, f32x16_t (&d)[TV][TB], int lane, At at) {
+  unsigned long long keep = 0;  // lanes whose row holds a NaN
+#pragma unroll
+  for (int tv = 0; tv < TV; ++tv) {
+    const f32x16_t& t = d[tv][TBI];
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) nan |= t[e] != t[e];
+    if (!__any(nan)) continue;
+#pragma unroll 1
+    for (int e = 0; e < 16; ++e) {  // wave-uniform: indexed registers
+      const float x = d[tv][TBI][e];
+      int b, v;
+      const bool live = at(tv, e, b, v);
+      unsigned long long todo = __ballot(live && x != x) & ~keep;
+      while (todo) {  // wave-uniform
+        const int row = __builtin_amdgcn_readlane(b, __builtin_ctzll(todo));
+        unsigned long long same = __ballot(b == row) & todo;
+        todo &= ~same;
+        if (row_has_nan(a, row, lane)) {
+          if (ROWLANE) keep |= __ballot(b == row);
+          continue;
+        }
+        for (; same; same &= same - 1) {
+          const int l = __builtin_ctzll(same);
+          const float s = wave_dot_f32(a, row, __builtin_amdgcn_readlane(v, l), lane);
+          d[tv][TBI][e] = lane == l ? s : d[tv][TBI][e];
+        }
+      }
+    }
+  }
+}
+// The maximum of column TBI of the wave's tiles; NaN if one of them is.
+template <int TBI, int TV, int TB>
+__device__ __forceinline__ float tile_max(const f32x16_t (&d)[TV][TB]) {
+  float m = d[0][TBI][0];
+#pragma unroll
+  for (int i = 1; i < TV * 16 - 1; i += 2)
+    m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, d[i / 16][TBI][i % 16]),
+                                      d[(i + 1) / 16][TBI][(i + 1) % 16]);
+  return __builtin_elementwise_maximum(m, d[TV - 1][TBI][15]);
+}
+
 // lm_head_ring.hip: one pass over W for up to kRingRows batch rows (sampling:
 // kRingSampleRows); 16-bit weight [V, H] and hidden of the same type, or bf16
 // weight and f32 hidden (kRingF32Rows), 16-byte aligned, H % 64 == 0

@@ -442,6 +442,20 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
   };
   auto epilogue = [&](int t) NVJSEL_INLINE {
     const int v0 = (blockIdx.x + t * gridDim.x) * BV + vi * 32 * TV;
+    if constexpr (NS == 3) {
+      auto redo = [&](auto TBI) NVJSEL_INLINE {
+        constexpr int tb = decltype(TBI)::value;
+        const float m = tile_max<tb>(acc);
+        if (__builtin_amdgcn_ballot_w64(m != m))
+          redo_nan_logits<tb, true>(a, acc, lane, [&](int tv, int e, int& b, int& v) NVJSEL_INLINE {
+            b = bj * 64 + tb * 32 + c32;
+            v = v0 + tv * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+            return b < B && v < V;
+          });
+      };
+      redo(std::integral_constant<int, 0>{});
+      redo(std::integral_constant<int, 1>{});
+    }
     if constexpr (SMP)
       sample_epilogue(v0);
     else

@@ -515,6 +515,16 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     const int t0 = tile_row(t);
     const int vend = min(tile_row(t + 1), r1);
     const int v0 = t0 + wv * TV * 32;
+    if constexpr (NS == 3) {
+      const float m = tile_max<0>(acc);
+      if (__builtin_amdgcn_ballot_w64(m != m))
+        redo_nan_logits<0, MODE != MODE_LOGITS>(a, acc, lane, [&](int tv, int e, int& b, int& v) NVJSEL_INLINE {
+          const int row = 8 * (e >> 2) + 4 * h + (e & 3);  // of D (logits: the batch row)
+          b = wb * 32 + (MODE == MODE_LOGITS ? row : c32);
+          v = v0 + tv * 32 + (MODE == MODE_LOGITS ? c32 : row);
+          return b < B && v < vend;
+        });
+    }
     if constexpr (MODE == MODE_LOGITS) {
       // operands swapped: D[batch 8 (e >> 2) + 4 h + (e & 3)][vocab c32], so
       // 32 lanes hold 32 consecutive logits of one row.  16-bit logits at

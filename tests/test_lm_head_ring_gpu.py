@@ -87,6 +87,48 @@ def test_ties_nan_and_infinities(reduce_cast):
     assert ids[1] == 777
 
 
+@pytest.mark.parametrize("B,H,V,layout", [
+    (20, 2048, 300, "vh"), (33, 64, 66000, "vh"), (64, 192, 257, "vh"),  # three terms in the staged GEMM
+    (200, 64, 515, "vh"),                                                # ... in the blocked GEMM
+    (20, 64, 1027, "hv"), (70, 128, 515, "hv"), (130, 64, 1027, "hv"), (200, 64, 520, "hv")])
+def test_f32_activations_keep_infinities(B, H, V, layout):
+    """f32 activations on bf16 weights give the logits of fp32 products where
+    an operand is infinite, a finite value rounds to bf16's infinity, or an
+    infinite weight meets a value whose lower terms are zero."""
+    rng = np.random.default_rng(B + H + V)
+    h = rng.standard_normal((B, H)).astype(np.float32)
+    w = (rng.standard_normal((V, H)) * 0.3).astype(np.float32)
+    h[0, 1] = np.inf
+    w[::7, 1] = 0.0  # inf * 0
+    h[1, 2] = -np.inf
+    h[2, 3] = 3.4e38
+    w[:, 3] *= 1e-3
+    h[3, 4], h[4, 4], h[5, 4], h[6, 4] = 1.0, 1.1, -0.7, 0.0
+    w[5, 4], w[9, 4] = np.inf, -np.inf
+    h[7, 5] = np.nan
+    wb = torch.from_numpy(w).cuda().to(torch.bfloat16)
+    hb = torch.from_numpy(h).cuda()
+    wo = wb if layout == "vh" else wb.T.contiguous()
+    h64, w64 = h.astype(np.float64), wb.float().cpu().numpy().astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        z = h64 @ w64.T
+        A = np.abs(h64) @ np.abs(w64).T
+    got = nvjsel.lm_head_logits_hip(hb, wo, weight_layout=layout).cpu().numpy().astype(np.float64)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(z))
+    fin = np.isfinite(z)
+    np.testing.assert_array_equal(got[~fin], z[~fin])
+    # fp32 sums of three products per element: 3 H 2^-24 sum |h w| at most
+    assert (np.abs(got[fin] - z[fin]) <= 3 * H * 2.0 ** -24 * A[fin]).all()
+    exp = np.where(np.isnan(z).any(axis=1), np.isnan(z).argmax(axis=1), np.nan_to_num(z, nan=0.0).argmax(axis=1))
+    ids, best = nvjsel.lm_head_greedy_top1_hip(hb, wo, weight_layout=layout, return_best=True)
+    np.testing.assert_array_equal(ids.cpu().numpy().reshape(-1), exp)  # (every row's best is not finite)
+    np.testing.assert_array_equal(best.cpu().numpy().astype(np.float64), z[np.arange(B), exp])
+    T = torch.tensor([float(b % 2) for b in range(B)]).cuda()
+    ids = nvjsel.lm_head_sample_token_ids(hb, wo, temperatures=T, rng_keys=keys_tensor(engine_keys(B, 3)),
+                                          weight_layout=layout)
+    np.testing.assert_array_equal(ids.cpu().numpy(), exp)  # an infinity or a NaN wins whatever the draw
+
+
 @pytest.mark.parametrize("B,H,layout", [(80, 64, "vh"), (40, 1024, "vh"), (20, 64, "hv"), (140, 64, "vh")])
 def test_sample_extreme_temperatures_and_nan(B, H, layout):
     """Tiny and huge temperatures (products with 1 / T' out of the float range
