@@ -1055,7 +1055,9 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
   // the chunk's L lanes that hold elements (ceil(k/4) in a full chunk).  The
   // waves then hold at least sum kk_w >= k lane maxima >= theta, so theta <=
   // the chunk's k-th largest logit.  Less a margin of 8 orderable units for
-  // values the division by T' may merge.
+  // values the division by T' may merge.  A chunk of fewer than k lanes (L <
+  // k) has no such floor: every element is a candidate, and a list that
+  // overflows sends the row to its exact path.
   const bool topk = rp.mode == ROW_FILTER && rp.k > 0 && rp.k <= kFastK;
   uint32_t wfloor = 0xFFFFFFFFu;
   if (topk && !wnan) {
@@ -1073,7 +1075,8 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     // prefix that kk lane maxima reach), the first lanes publish the
     // largest lane maxima, lane kTops-1 the kTops-th (-inf fills)
     const uint32_t sk = wave_sort_desc(r.vok[0] ? radix_key(tv) : 0u);
-    wfloor = kk ? ((uint32_t)__builtin_amdgcn_readlane((int)sk, (int)kk - 1) >> 16) << 16 : 0xFFFFFFFFu;
+    const bool some = kk <= (uint32_t)Lw;  // (kk - 1 is a lane: at most 63)
+    wfloor = !kk ? 0xFFFFFFFFu : some ? ((uint32_t)__builtin_amdgcn_readlane((int)sk, (int)kk - 1) >> 16) << 16 : 0u;
     const float sv = sk > 0x007FFFFFu ? radix_value(sk) : -INFINITY;
     float* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
     if (lane < 1 << tops_shift(a)) tops[lane] = sv;
@@ -1515,7 +1518,7 @@ __global__ void __launch_bounds__(kThreads) topk_select_kernel(SampleArgs a, flo
     fast = !__syncthreads_or(bad);
     if (fast) {
       n = load_candidates(a, b, row_params(a, b), s.off, (int)tot, s.cand, kSelCap, &s.n, s.red);
-      fast = n <= kSelCap;
+      fast = n >= K && n <= kSelCap;  // (n >= K: no floor lies above the row's k-th largest)
     }
   }
   int m = K;  // entries of s.sel to sort

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("V", [300, 8192, 16385, 37888, 50257, 65536, 131072])
+@pytest.mark.parametrize("V", [300, 1000, 8192, 16385, 37888, 50257, 65536, 131072])
 def test_top_k_rows(V, dtype):
     rng = np.random.default_rng(V)
     ks = [20, 100, 100, 128, 200, 256]

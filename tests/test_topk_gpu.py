@@ -36,6 +36,18 @@ def test_topk_random(dt, batch, vocab, k):
     _check(x, k, f"{dt} B={batch} V={vocab} k={k}")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("vocab", [300, 504, 1000, 16384 + 40, 66000])
+def test_topk_more_than_a_chunks_lanes(dt, vocab):
+    """k above the lanes that hold elements of a row's only or last chunk: that
+    many lane maximums, which bound the k-th largest, do not exist."""
+    g = torch.Generator().manual_seed(vocab)
+    x = (torch.randn(8, vocab, generator=g) * 3).to(TORCH[dt])
+    x[4:, -40:] += 6.0  # the short chunk holds the largest
+    for k in (100, 126, 130, 200, 256):
+        _check(x.cuda(), k, f"{dt} V={vocab} k={k}")
+
+
 def test_topk_zipf_rows_real_fixture():
     d = np.load("tests/golden/qwen08_logits_row.npz")
     row = torch.from_numpy(np.asarray(d["logits_0"], np.float32)).reshape(1, -1)
