@@ -13,20 +13,19 @@ namespace nvjsel {
 // floor does) and from 16 nc = 9/8 k on: those rows want nothing more, and
 // publishing or listing more for them only costs (k = 256 at 31 chunks 37 us
 // against 58 with tier B).  Below, eight maximums per wave settle the row
-// where 32 nc >= 5/4 k; tier B (the lists down to the chunk's own floor) where
-// the floor is a published value or few chunks hold the row and the lists stay
-// within their 512 entries.  Elsewhere (k = 256 below 10 chunks, k = 160 at
-// two) nothing helps and the descent is not delayed by it (54 us against 71).
+// where 32 nc >= 7/5 k (the last chunk may hold little); tier B (the lists down
+// to the chunk's own floor) where 32 nc >= 6/5 k, or few chunks hold the row,
+// and the lists stay within their 512 entries.  Elsewhere (k = 256 below 12
+// chunks, k = 160 at two, 200 at one) most rows would still miss, and their
+// descent is not delayed by it
+// (k = 256 at one chunk 55 us against 71 with tier B).
 // V = 50,257 / 98,304, k = 100, 64 rows: 270 / 413 -> 51 / 31 us.
 constexpr bool topk_floor_low(int nc, int k) { return k > 32 && 128 * nc < 9 * k; }
 constexpr bool topk_tier_b(int nc, int k) {
-  return topk_floor_low(nc, k) && k <= 200 && 64 * nc < 3 * k && (32 * nc >= k || nc * k <= 300);
+  return topk_floor_low(nc, k) && 64 * nc < 3 * k && (160 * nc >= 6 * k ? k <= 200 : k <= 160 && nc * k <= 300);
 }
-// (select reads the second four with the row's other words, before it knows
-// k: on 13 and more chunks that slowed the rows that do not need them by 0.6-1%)
-constexpr int kTopsMoreChunks = 13;
 constexpr bool topk_more_tops(int nc, int k) {
-  return nc < kTopsMoreChunks && topk_floor_low(nc, k) && (128 * nc >= 5 * k || topk_tier_b(nc, k));
+  return topk_floor_low(nc, k) && (160 * nc >= 7 * k || topk_tier_b(nc, k));
 }
 
 }  // namespace nvjsel

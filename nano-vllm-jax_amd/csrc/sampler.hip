@@ -46,6 +46,7 @@
 #include <climits>
 #include "nvjsel_device.h"
 #include "nvjsel_host.h"
+#include "route_rules.h"
 
 namespace nvjsel {
 
@@ -99,7 +100,8 @@ struct SampleArgs {
   float* cand_floor_a;             // [B, nchunks]
   float* cand_floor;               // [B, nchunks] logit floor of each chunk's candidates
   unsigned long long* cand;        // [B, nchunks, kCandCap]; one-pass calls: [B, sub-chunks] block keys
-  uint32_t* topp_chunk_hist;       // [B, nchunks, kToppBins] chunk histograms, 2^-17 units (top-p-only rows)
+  uint32_t* topp_chunk_hist;       // [B, nchunks, kToppBins] chunk histograms, 2^-17 units (top-p-only rows);
+                                   // top-k rows: the second four lane maxima of each wave (topk_more_tops)
   int32_t* topp_chunk_tb;          // [B, nchunks] grid bin of each chunk's maximum
   int32_t* row_ib;                 // [B] top-p rows: grid bin of the crossing (INT_MIN: none)
   unsigned long long* row_target;  // [B] top-p rows: weight units needed inside the crossing bin
@@ -596,11 +598,12 @@ __device__ __forceinline__ unsigned long long wave_gumbel(const SampleArgs& a, i
 
 // ------------------------------------------------------------------ top-k rows from candidates
 // A FILTER row with k <= 256: the row floor is the larger of the largest chunk
-// floor and the k-th largest lane maximum the scan published (tops_shift);
+// floor and the k-th largest lane maximum the scan published (four per wave,
+// or eight: topk_more_tops);
 // the candidates at or above it (about k of them) are rank-sorted in LDS, and
 // top-k, top-p and the exact Gumbel-max read the sorted prefix.
 static constexpr int kTops = 8;        // lane maxima ranked per wave (tier A bound)
-static constexpr int kTopsPub = 8;     // most of them published per wave (row floor)
+static constexpr int kTopsPub = 4;     // of them published per wave (row floor), twice as many where topk_more_tops
 static constexpr int kTopsChunks = 64; // chunks whose tops bound the row floor (<= 1024 values)
 static constexpr int kFinCap = 512;    // survivors sorted in LDS
 
@@ -616,20 +619,13 @@ struct FinishShared {
   uint32_t n, kf, tau, rem, nk;
 };
 
-// log2 of the lane maximums published per wave: eight on fewer than 13 chunks,
-// where four per wave are fewer than twice a k of 100, else four (V = 50,257, k
-// = 100 at 7 chunks 197 -> 33 us; reading eight slowed mixed calls at 14 and
-// 16 chunks by 0.6-1%).
-__device__ __forceinline__ int tops_shift(const SampleArgs& a) { return a.nchunks < 13 ? 3 : 2; }
-
-// Whether the scan writes a top-k row's tier B too: always for nvjsel_topk; for
-// the sampler where the row's chunks hold so few of the k that some chunk's
-// tier A (at least 32 elements) may end above the row floor, which is the k-th
-// of the lane maximums the chunks publish (k = 100 below 7 chunks).  A row
-// whose lists stop short takes a whole-row descent: V = 37,888, 67 rows, k =
-// 100 152 us against 26-39.
+// Whether the scan writes a top-k row's tier B too: always for nvjsel_topk.
 __device__ __forceinline__ bool scan_tier_b(const SampleArgs& a, const RowParams& rp) {
-  return a.topk > 0 || ((kThreads / 64) * a.nchunks << tops_shift(a)) < 2 * rp.k;
+  return a.topk > 0 || topk_tier_b(a.nchunks, rp.k);
+}
+// Chunk c's second four lane maxima per wave (16 floats).
+__device__ __forceinline__ float* more_tops(const SampleArgs& a, int b, int c) {
+  return (float*)(a.topp_chunk_hist + ((size_t)b * a.nchunks + c) * kToppBins);
 }
 
 // The first loads of a fast top-k row, issued by select before it reduces the
@@ -656,13 +652,12 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPr
     pf.fl_a = a.cand_floor_a[i];
     pf.fl = a.cand_floor[i];
   }
-  const int ts = tops_shift(a);
-  const int nvals = (min(NC, kTopsChunks) * (kThreads / 64)) << ts;
+  const int nvals = min(NC, kTopsChunks) * (kThreads / 64) * kTopsPub;
   const float* tops = a.lane_tops + (size_t)b * NC * (kThreads / 64) * kTopsPub;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = (int)threadIdx.x + kThreads * i;
-    pf.key[i] = j < nvals ? radix_key(tops[(j >> ts) * kTopsPub + (j & ((1 << ts) - 1))]) >> 16 : 0u;
+    pf.key[i] = j < nvals ? radix_key(tops[j]) >> 16 : 0u;
   }
   // the first list entries the gather reads, requested now rather than once
   // the row floor is known (inside each chunk's list area; entries past the
@@ -718,7 +713,17 @@ __device__ int topk_sorted_survivors(const SampleArgs& a, int b, const RowParams
     s.cnt_a[threadIdx.x] = pf.cnt_a;
     s.fl_a[threadIdx.x] = pf.fl_a;
   }
-  const uint32_t kf16 = row_tops_kth(pf.key, rp.k, s) << 16;
+  uint32_t keys[4] = {pf.key[0], pf.key[1], pf.key[2], pf.key[3]};
+  if (__builtin_expect(topk_more_tops(NC, rp.k), 0)) {
+    // (at most 17 chunks, 272 values each way: keys[2] and [3] are free.  Read
+    // here, not with the prefetched words: rows without them need no other load)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int j = (int)threadIdx.x + kThreads * i;
+      if (j < NC * (kThreads / 64) * kTopsPub) keys[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
+    }
+  }
+  const uint32_t kf16 = row_tops_kth(keys, rp.k, s) << 16;
   if (threadIdx.x == 0) s.n = 0;
   const float flmax = unord_f32((uint32_t)block_max_u64(ord_f32(pf.fl), s.red));  // (barriers)
   // the row floor (raw logits) and, per chunk, how much of its list can reach it
@@ -1072,18 +1077,22 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     // the lane maxima as radix keys (lanes holding no element of the row: 0,
     // below every value), sorted: lane t holds the t-th largest.  The
     // kk-th largest gives the wave floor (its top 16 bits: the largest
-    // prefix that kk lane maxima reach), the first lanes publish the
+    // prefix that kk lane maxima reach), lanes 0..kTopsPub-1 publish the
     // largest lane maxima, lane kTops-1 the kTops-th (-inf fills)
     const uint32_t sk = wave_sort_desc(r.vok[0] ? radix_key(tv) : 0u);
     const bool some = kk <= (uint32_t)Lw;  // (kk - 1 is a lane: at most 63)
     wfloor = !kk ? 0xFFFFFFFFu : some ? ((uint32_t)__builtin_amdgcn_readlane((int)sk, (int)kk - 1) >> 16) << 16 : 0u;
     const float sv = sk > 0x007FFFFFu ? radix_value(sk) : -INFINITY;
     float* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
-    if (lane < 1 << tops_shift(a)) tops[lane] = sv;
+    if (lane < kTopsPub) tops[lane] = sv;
+    if (__builtin_expect(topk_more_tops(a.nchunks, rp.k), 0)) {
+      if (lane >= kTopsPub && lane < 2 * kTopsPub) more_tops(a, b, c)[wave * kTopsPub + lane - kTopsPub] = sv;
+    }
     if (lane == kTops - 1) sh.wtop[wave] = sv;
   } else if (topk && lane < kTopsPub) {
     if (lane == 0) sh.wtop[wave] = -INFINITY;
     a.lane_tops[(((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub + lane] = -INFINITY;
+    if (topk_more_tops(a.nchunks, rp.k)) more_tops(a, b, c)[wave * kTopsPub + lane] = -INFINITY;
   }
   if (lane == 0) { sh.wkey[wave] = wkey; sh.wfloor[wave] = wfloor; }
   if (threadIdx.x == 0) { sh.cnt = 0; sh.cnt_b = 0; sh.waves = 0; }
@@ -1143,8 +1152,9 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
   // Tier A, written first: candidates at or above t_a = min over waves of the
   // wave's kTops-th largest lane maximum (the chunk holds at least
   // 4 * kTops elements >= t_a).  A row floor >= t_a needs only tier A; tier B,
-  // the rest down to theta, is written where the floor may lie lower
-  // (scan_tier_b; elsewhere the rare row that needs it takes the exact path).
+  // the rest down to theta, is written where the floor lies lower and the
+  // lists can hold it (scan_tier_b; elsewhere a row that needs it takes the
+  // exact path).
   float t_a = sh.wtop[0];
 #pragma unroll
   for (int w = 1; w < kThreads / 64; ++w) t_a = fminf(t_a, sh.wtop[w]);
