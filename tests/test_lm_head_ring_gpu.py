@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import nvjsel
+from nvjsel import _lib
 from oracle import selection as sel
 from tests.gpu_helpers import check_fused_sampled, check_greedy, engine_keys, keys_tensor
 
@@ -46,6 +47,30 @@ def test_greedy_and_logits(B, H, V, dt):
     # the winning logit is the row's largest stored logit, at its first index
     np.testing.assert_array_equal(best.cpu().numpy(), logits.float().max(dim=1).values.cpu().numpy())
     np.testing.assert_array_equal(ids.cpu().numpy().reshape(-1), got.argmax(axis=1))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,stride,base", [(516, 516, 0), (516, 520, 4), (516, 517, 0), (516, 518, 0), (516, 516, 1),
+                                           (516, 516, 2), (514, 516, 0), (515, 515, 0), (2052, 2053, 3)])
+def test_logits_row_stride_and_base(V, stride, base, dt):
+    """16-bit logits leave 8 bytes per lane only where every row's quads allow
+    it; other strides and bases store the same values, and nothing is written
+    between the rows.  base: elements past a 256-byte boundary."""
+    B, H = 45, 64
+    _, h, w, z, rc = _inputs(B, H, V, dt, 2)
+    code = _lib.BF16 if dt == torch.bfloat16 else _lib.F16
+    buf = torch.full((base + B * stride + 8,), -777.0, device="cuda", dtype=dt)
+    _lib.call("nvjsel_lm_head_logits", h.data_ptr(), code, w.data_ptr(), code, _lib.W_VH, B, H, V, rc,
+              buf.data_ptr() + 2 * base, code, stride, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    rows = buf[base:base + B * stride].view(B, stride)
+    assert bool((buf[:base] == -777.0).all()) and bool((buf[base + B * stride:] == -777.0).all())
+    assert bool((rows[:, V:] == -777.0).all())
+    torch.testing.assert_close(rows[:, :V], nvjsel.lm_head_logits_hip(h, w, weight_layout="vh"), rtol=0, atol=0)
+    hn = np.linalg.norm(h.float().cpu().numpy(), axis=1)[:, None]
+    wn = np.linalg.norm(w.float().cpu().numpy(), axis=1)[None, :]
+    tol = H * 2.0 ** -23 * hn * wn + np.abs(z) * {1: 2.0 ** -8, 2: 2.0 ** -11}[rc] + 1e-7  # as above
+    assert (np.abs(rows[:, :V].float().cpu().numpy().astype(np.float64) - z) <= tol).all()
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
