@@ -454,12 +454,15 @@ __global__ void __launch_bounds__(kGemvWaves * 64) lm_head_gemv_kernel(LmArgs a)
 // KU rows are in flight per wave; acc[b][c] += h[b][k] * W[k][col + c] in
 // fp32, with h broadcast from LDS.  The slices' partial sums meet in LDS,
 // summed in slice order, and each thread then scores two columns of every row.
-// Any V >= 8: rows start at any element, so the loads are 16 bytes from any
-// element address (one instruction; V = 50,257, H = 768, B = 4 sampled 1700 ->
-// 23 us against one thread per column).  A group that ends past its row reads on
-// into the next one (those columns are never scored); in the last row it is
-// loaded from V - 8 and moved down.
-template <int WT, int NB, int WAVES, int MODE, bool DOTP>
+// VEC8: rows of whole, aligned 16-byte groups (V % 8 == 0).  Else any V >= 8:
+// rows start at any element, so the loads are 16 bytes from any element
+// address (one instruction; V = 50,257, H = 768, B = 4 sampled 1700 -> 23 us
+// against one thread per column).  A group that ends past its row reads on into
+// the next one (those columns are never scored); in the last row it is loaded
+// from V - 8 and moved down.  One body for both cost the aligned rows up to 50%
+// (V = 32,000, H = 1024, f32 B = 1 / 8 38.9 / 72.8 us against 29.1 / 63.8; V =
+// 98,304, bf16 B = 8 46.7 against 42.9).
+template <int WT, int NB, int WAVES, int MODE, bool DOTP, bool VEC8>
 __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
   // DOT (bf16 hidden, a k-slice of even length): the hidden sits in LDS as
   // bf16 pairs (k, k+1) and each pair of W rows is packed per column with
@@ -474,8 +477,9 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int H = a.H, V = a.V, B = a.B;
   const int vb = blockIdx.x * STRIP;
-  const int col = vb + lane * 8 < V ? vb + lane * 8 : V - 8;  // groups wholly past the row end: any columns
-  const int over = max(col - (V - 8), 0);  // elements of the group past the row end
+  // groups wholly past the row end: any columns (VEC8: the last group)
+  const int col = VEC8 ? min(vb + lane * 8, V - 8) : vb + lane * 8 < V ? vb + lane * 8 : V - 8;
+  const int over = VEC8 ? 0 : max(col - (V - 8), 0);  // elements of the group past the row end
   if constexpr (DOT) {
     uint32_t* lds_p = (uint32_t*)lds_f;  // [H / 2][NB] bf16 pairs
     const uint16_t* hs = (const uint16_t*)a.hidden;
@@ -518,8 +522,12 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
           const int k = min(k0 + j * KU + u, k1 - 1);
-          const int c = k == H - 1 ? col - over : col;
-          ring[decltype(S)::value][u] = __builtin_nontemporal_load((const u32x4_any_t*)(W + (size_t)k * V + c));
+          if constexpr (VEC8) {
+            ring[decltype(S)::value][u] = stream_load((const u32x4_t*)(W + (size_t)k * V + col));
+          } else {
+            const int c = k == H - 1 ? col - over : col;
+            ring[decltype(S)::value][u] = __builtin_nontemporal_load((const u32x4_any_t*)(W + (size_t)k * V + c));
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       },
@@ -530,7 +538,7 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
             const int k = k0 + i * KU + u;
             if (k >= k1) continue;  // wave-uniform; the slice length is even
             u32x4_t w0 = ring[decltype(S)::value][u], w1 = ring[decltype(S)::value][u + 1];
-            if (k + 1 == H - 1) w1 = shift_down8(w1, over);  // (H is even)
+            if (!VEC8 && k + 1 == H - 1) w1 = shift_down8(w1, over);  // (H is even)
             const uint32_t q0[4] = {w0.x, w0.y, w0.z, w0.w}, q1[4] = {w1.x, w1.y, w1.z, w1.w};
             uint32_t wp[8];  // column c: (W[k][c], W[k+1][c]) as a bf16 pair
 #pragma unroll
@@ -554,7 +562,7 @@ __global__ void __launch_bounds__(WAVES * 64) lm_head_hv_kernel(LmArgs a) {
           const int k = k0 + i * KU + u;
           if (k >= k1) continue;  // wave-uniform (last step of the slice)
           u32x4_t w = ring[decltype(S)::value][u];
-          if (k == H - 1) w = shift_down8(w, over);
+          if (!VEC8 && k == H - 1) w = shift_down8(w, over);
           const uint32_t q[4] = {w.x, w.y, w.z, w.w};
           float wf[8];
 #pragma unroll
@@ -1221,9 +1229,13 @@ struct LogitsOut {
 template <int WT, int NB, int MODE>
 static int launch_hv(const LmArgs& a, hipStream_t stream) {
   constexpr int WAVES = 4;  // measured: 4 waves per block beat 8 and 16 at B = 1 and 8
-  auto kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, false>;
+  auto kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, false, false>;
   if constexpr (WT == DT_BF16) {
-    if (kHvDot && a.hidden_dtype == DT_BF16 && (a.H % (2 * WAVES)) == 0) kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, true>;
+    const bool vec8 = (a.V % 8) == 0 && (((uintptr_t)a.W) & 15) == 0;
+    if (kHvDot && a.hidden_dtype == DT_BF16 && (a.H % (2 * WAVES)) == 0)
+      kern = vec8 ? lm_head_hv_kernel<WT, NB, WAVES, MODE, true, true> : lm_head_hv_kernel<WT, NB, WAVES, MODE, true, false>;
+    else if (vec8)
+      kern = lm_head_hv_kernel<WT, NB, WAVES, MODE, false, true>;
   }
   const size_t lds = hv_lds_bytes(NB, a.H);
   if (lds > 48 * 1024)

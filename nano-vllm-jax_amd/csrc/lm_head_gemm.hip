@@ -127,11 +127,14 @@ __device__ __forceinline__ void gemm_finish_rows(const LmArgs& a, unsigned long 
 // NARROW: B <= 64; each wave owns 32 vocabulary rows x the 64 batch rows
 // (instead of 128 x 64 of one batch quarter), so all 8 waves multiply and,
 // in sample mode, draw.
-// WT: weight (and NS = 1: hidden) element type.  [H, V] rows start at any
-// element (V >= 8): 16-byte loads from element addresses; a group that ends
-// past its row reads on into the next one (columns masked where they could
-// win), in the last row it is loaded from V - 8 and moved down as it is stored.
-template <int WT, int MODE, int BV, int NS, int KC, bool HV, bool PART, bool NARROW>
+// WT: weight (and NS = 1: hidden) element type.  VEC8: [H, V] rows of whole,
+// aligned 16-byte groups (V % 8 == 0); groups past the row end re-read the last
+// one.  Else rows start at any element (V >= 8): 16-byte loads from element
+// addresses; a group that ends past its row reads on into the next one (columns
+// masked where they could win), in the last row it is loaded from V - 8 and
+// moved down as it is stored: 2-4% more time on aligned rows (f32 hidden, V =
+// 32,000, H = 1024, B = 32 48.8 us against 47.6).
+template <int WT, int MODE, int BV, int NS, int KC, bool HV, bool VEC8, bool PART, bool NARROW>
 __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a) {
   constexpr int Q = KC / 8;  // 8-element columns per row and stage
   static_assert(!(PART && NARROW), "one batch layout");
@@ -220,7 +223,10 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
     stage_of(st, v0, kc);
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
-      if constexpr (HV) {
+      if constexpr (HV && VEC8) {
+        const int v = min(v0 + aq[i] * 8, V - 8);
+        RA[e][i] = *(const u32x4_t*)(W + (size_t)(kc * KC + arow[i]) * V + v);
+      } else if constexpr (HV) {
         const int k = kc * KC + arow[i];
         const int v = v0 + aq[i] * 8 < V ? v0 + aq[i] * 8 : V - 8;
         over[e][i] = k == H - 1 ? max(v - (V - 8), 0) : 0;
@@ -245,7 +251,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
     constexpr int e = decltype(set)::value, f = decltype(buf)::value;
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
-      if constexpr (HV) {
+      if constexpr (HV && !VEC8) {
         if (__any(over[e][i])) RA[e][i] = shift_down8(RA[e][i], over[e][i]);
       }
       As[f][aslot[i]] = RA[e][i];
@@ -530,7 +536,7 @@ __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a
 // 185 us at B = 256, V = 248320) or 128 (4 waves, two blocks per CU: 195 us)
 static constexpr int kGemmBV = 256;
 static constexpr int kGemmBpc = 256 / kGemmBV;  // blocks per CU of the blocked GEMM
-template <int WT, int MODE, int NS, bool HV>
+template <int WT, int MODE, int NS, bool HV, bool VEC8>
 static int launch_gemm_shape(const LmArgs& a, hipStream_t stream) {
   const int ntiles = (a.V + kGemmBV - 1) / kGemmBV;
   int grid = kGemmBpc * device_cu_count();
@@ -541,7 +547,7 @@ static int launch_gemm_shape(const LmArgs& a, hipStream_t stream) {
   constexpr bool kNarrow = HV;
   if constexpr (kNarrow) {
     if (a.B <= 64) {
-      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, kGemmKC, HV, false, true>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, kGemmKC, HV, VEC8, false, true>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
       NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
       return NVJSEL_OK;
     }
@@ -551,12 +557,12 @@ static int launch_gemm_shape(const LmArgs& a, hipStream_t stream) {
   } else {
     if constexpr (HV || NS == 1) {  // ([V, H] f32 passes of <= 192 rows take the staged GEMM)
       if (a.B <= kGemmBB - 64) {
-        hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, true, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+        hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, VEC8, true, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
         NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
         return NVJSEL_OK;
       }
     }
-    hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, false, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+    hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, KC, HV, VEC8, false, false>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
   }
   NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
   return NVJSEL_OK;
@@ -569,17 +575,25 @@ int launch_gemm(int mode, bool hv, const LmArgs& a, hipStream_t stream) {
     return fn(std::integral_constant<int, MODE_LOGITS>{});
   };
   if (!hv && a.hidden_dtype == DT_F32)
-    return by_mode([&](auto M) { return launch_gemm_shape<DT_BF16, decltype(M)::value, 3, false>(a, stream); });
+    return by_mode([&](auto M) { return launch_gemm_shape<DT_BF16, decltype(M)::value, 3, false, false>(a, stream); });
   if (!hv) {
     if (mode != MODE_SAMPLE || a.hidden_dtype != DT_BF16)
       return fail(NVJSEL_EINVAL, "launch_gemm: [V, H] weights take the staged GEMM");
-    return launch_gemm_shape<DT_BF16, MODE_SAMPLE, 1, false>(a, stream);
+    return launch_gemm_shape<DT_BF16, MODE_SAMPLE, 1, false, false>(a, stream);
   }
-  if (a.hidden_dtype == DT_F32)
-    return by_mode([&](auto M) { return launch_gemm_shape<DT_BF16, decltype(M)::value, 3, true>(a, stream); });
+  // (f16 weights take the any-element loads: their rows were never faster)
+  const bool vec8 = (a.V % 8) == 0 && (((uintptr_t)a.W) & 15) == 0;
   if (a.weight_dtype == DT_F16)
-    return by_mode([&](auto M) { return launch_gemm_shape<DT_F16, decltype(M)::value, 1, true>(a, stream); });
-  return by_mode([&](auto M) { return launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true>(a, stream); });
+    return by_mode([&](auto M) { return launch_gemm_shape<DT_F16, decltype(M)::value, 1, true, false>(a, stream); });
+  if (a.hidden_dtype == DT_F32)
+    return by_mode([&](auto M) {
+      return vec8 ? launch_gemm_shape<DT_BF16, decltype(M)::value, 3, true, true>(a, stream)
+                  : launch_gemm_shape<DT_BF16, decltype(M)::value, 3, true, false>(a, stream);
+    });
+  return by_mode([&](auto M) {
+    return vec8 ? launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true, true>(a, stream)
+                : launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true, false>(a, stream);
+  });
 }
 
 }  // namespace nvjsel
