@@ -4,28 +4,32 @@
 
 namespace nvjsel {
 
-// ---- top-k rows of the sampler (k <= 256) on `nc` scan chunks of four waves.
-// Each wave publishes its four largest lane maximums and each chunk lists its
-// elements down to tier A (at least 32 of them); a row is settled from the
-// lists if the row floor -- the larger of the k-th of the 16 nc published
-// values and the largest chunk floor -- reaches every chunk's tier A, and
-// takes a whole-row descent if not.  That holds for k <= 32 (a chunk's own
-// floor does) and from 16 nc = 9/8 k on: those rows want nothing more, and
-// publishing or listing more for them only costs (k = 256 at 31 chunks 37 us
-// against 58 with tier B).  Below, eight maximums per wave settle the row
-// where 32 nc >= 7/5 k (the last chunk may hold little); tier B (the lists down
-// to the chunk's own floor) where 32 nc >= 6/5 k, or few chunks hold the row,
-// and the lists stay within their 512 entries.  Elsewhere (k = 256 below 12
-// chunks, k = 160 at two, 200 at one) most rows would still miss, and their
-// descent is not delayed by it
-// (k = 256 at one chunk 55 us against 71 with tier B).
-// V = 50,257 / 98,304, k = 100, 64 rows: 270 / 413 -> 51 / 31 us.
-constexpr bool topk_floor_low(int nc, int k) { return k > 32 && 128 * nc < 9 * k; }
-constexpr bool topk_tier_b(int nc, int k) {
-  return topk_floor_low(nc, k) && 64 * nc < 3 * k && (160 * nc >= 6 * k ? k <= 200 : k <= 160 && nc * k <= 300);
-}
-constexpr bool topk_more_tops(int nc, int k) {
-  return topk_floor_low(nc, k) && (160 * nc >= 7 * k || topk_tier_b(nc, k));
+// ---- top-k rows of the sampler (k <= 256) on `nc` scan chunks of four waves,
+// the last one `fill` eighths full (1-8).  Each wave publishes its four largest
+// lane maximums and each chunk lists its elements down to tier A (at least 32
+// of them); a row is settled from the lists if the row floor -- the larger of
+// the k-th of the 16 nc published values and the largest chunk floor -- reaches
+// every chunk's tier A, and takes a whole-row descent if not (64 f32 rows at 10
+// chunks 380 us against 25).  k <= 32 rows always settle (a chunk's own floor
+// does); the others want twice the published values until 16 nc = 7/5 k (one
+// more load: no measured cost), and below 16 nc = k tier B, the lists down to
+// the chunk's own floor (k = 128-160 rows 31 us with it where they settle
+// without, 26), as long as its floors come out high enough:
+//  * from the published values, once 32 nc (counting the last chunk's fill)
+//    reaches 0.88 k, 1.16 k above 160 (k = 160 at 4.25 / 5 chunks 187 / 51 us
+//    with, 172 / 196 without; k = 200 at 6.25 / 9 253 / 37 and 240 / 441), and
+//  * from a single chunk's, while the survivors stay below 512: k = 128 at 2 /
+//    2.25 / 2.6 chunks 40 / 93 / 127 us with, 97 / 106 / 118 without; k = 160 at
+//    1.25 / 1.6 chunks 43 / 94 and 75 / 87.
+// Above k = 200 the lists hold tier B only just before nothing needs it (k =
+// 256 at 12 chunks of 16 bits 52 us with, 230 without; at 11 434 and 430).
+constexpr bool topk_more_tops(int nc, int k) { return k > 32 && k <= 256 && 80 * nc < 7 * k; }
+constexpr bool topk_tier_b(int nc, int k, int fill) {
+  if (k <= 32 || 16 * nc >= k) return false;
+  const int e = 8 * (nc - 1) + fill;  // the row in eighths of a chunk
+  if (k <= 160) return 50 * e >= 11 * k || e * k <= (k <= 128 ? 2400 : 1600);
+  if (k <= 200) return 100 * e >= 29 * k;
+  return 200 * e >= 73 * k && 1600 * nc <= 82 * k;
 }
 
 }  // namespace nvjsel

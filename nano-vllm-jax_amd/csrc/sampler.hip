@@ -83,6 +83,7 @@ struct SampleArgs {
   int V;
   int nchunks;
   int chunk;  // elements per scan chunk (256 * EPT)
+  int last_fill;  // eighths of the last chunk that hold elements (1-8)
   long long stride;  // elements between rows
   const float* temperature;
   const int32_t* top_k;
@@ -100,8 +101,7 @@ struct SampleArgs {
   float* cand_floor_a;             // [B, nchunks]
   float* cand_floor;               // [B, nchunks] logit floor of each chunk's candidates
   unsigned long long* cand;        // [B, nchunks, kCandCap]; one-pass calls: [B, sub-chunks] block keys
-  uint32_t* topp_chunk_hist;       // [B, nchunks, kToppBins] chunk histograms, 2^-17 units (top-p-only rows);
-                                   // top-k rows: the second four lane maxima of each wave (topk_more_tops)
+  uint32_t* topp_chunk_hist;       // [B, nchunks, kToppBins] chunk histograms, 2^-17 units (top-p-only rows)
   int32_t* topp_chunk_tb;          // [B, nchunks] grid bin of each chunk's maximum
   int32_t* row_ib;                 // [B] top-p rows: grid bin of the crossing (INT_MIN: none)
   unsigned long long* row_target;  // [B] top-p rows: weight units needed inside the crossing bin
@@ -621,11 +621,13 @@ struct FinishShared {
 
 // Whether the scan writes a top-k row's tier B too: always for nvjsel_topk.
 __device__ __forceinline__ bool scan_tier_b(const SampleArgs& a, const RowParams& rp) {
-  return a.topk > 0 || topk_tier_b(a.nchunks, rp.k);
+  return a.topk > 0 || topk_tier_b(a.nchunks, rp.k, a.last_fill);
 }
-// Chunk c's second four lane maxima per wave (16 floats).
+// Chunk c's second four lane maxima per wave (16 floats): the last eight entries
+// of its list, whose page scan and select touch anyway.
+static constexpr int kMoreTops = 8;
 __device__ __forceinline__ float* more_tops(const SampleArgs& a, int b, int c) {
-  return (float*)(a.topp_chunk_hist + ((size_t)b * a.nchunks + c) * kToppBins);
+  return (float*)(a.cand + ((size_t)b * a.nchunks + c) * kCandCap + (kCandCap - kMoreTops));
 }
 
 // The first loads of a fast top-k row, issued by select before it reduces the
@@ -635,11 +637,11 @@ __device__ __forceinline__ float* more_tops(const SampleArgs& a, int b, int c) {
 struct TopkPrefetch {
   uint32_t cnt, cnt_a;
   float fl_a, fl;
-  uint32_t key[4];  // published lane maxima t + 256 i, as 16-bit keys (0: none)
+  uint32_t key[4];  // published lane maxima t + 256 i, as 16-bit keys (0: none); [2], [3]: topk_more_tops
   unsigned long long cv[4];  // entries (t & 7) + 8 q of chunk t >> 3's list (the gather's first reads)
 };
 
-__device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPrefetch& pf) {
+__device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, int k, TopkPrefetch& pf) {
   const int NC = a.nchunks;
   pf.cnt = 0;
   pf.cnt_a = 0;
@@ -666,6 +668,15 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPr
   const unsigned long long* src = a.cand + ((size_t)b * NC + (c < NC ? c : 0)) * kCandCap;
 #pragma unroll
   for (int q = 0; q < 4; ++q) pf.cv[q] = src[(threadIdx.x & 7) + 8 * q];
+  // last, and only for rows that want them: read for every row (so that they
+  // need not wait for k) they cost k = 20 rows 0.3 us
+  if (topk_more_tops(NC, k)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // (key[2] and [3] are free: k <= 256, so 16 NC <= 352; other rows drop them)
+      const int j = (int)threadIdx.x + kThreads * i;
+      if (j < NC * (kThreads / 64) * kTopsPub) pf.key[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
+    }
+  }
 }
 
 // Largest 16-bit prefix p with at least k of the row's published lane maxima
@@ -713,17 +724,7 @@ __device__ int topk_sorted_survivors(const SampleArgs& a, int b, const RowParams
     s.cnt_a[threadIdx.x] = pf.cnt_a;
     s.fl_a[threadIdx.x] = pf.fl_a;
   }
-  uint32_t keys[4] = {pf.key[0], pf.key[1], pf.key[2], pf.key[3]};
-  if (__builtin_expect(topk_more_tops(NC, rp.k), 0)) {
-    // (at most 17 chunks, 272 values each way: keys[2] and [3] are free.  Read
-    // here, not with the prefetched words: rows without them need no other load)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int j = (int)threadIdx.x + kThreads * i;
-      if (j < NC * (kThreads / 64) * kTopsPub) keys[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
-    }
-  }
-  const uint32_t kf16 = row_tops_kth(keys, rp.k, s) << 16;
+  const uint32_t kf16 = row_tops_kth(pf.key, rp.k, s) << 16;
   if (threadIdx.x == 0) s.n = 0;
   const float flmax = unord_f32((uint32_t)block_max_u64(ord_f32(pf.fl), s.red));  // (barriers)
   // the row floor (raw logits) and, per chunk, how much of its list can reach it
@@ -1085,7 +1086,7 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     const float sv = sk > 0x007FFFFFu ? radix_value(sk) : -INFINITY;
     float* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
     if (lane < kTopsPub) tops[lane] = sv;
-    if (__builtin_expect(topk_more_tops(a.nchunks, rp.k), 0)) {
+    if (topk_more_tops(a.nchunks, rp.k)) {
       if (lane >= kTopsPub && lane < 2 * kTopsPub) more_tops(a, b, c)[wave * kTopsPub + lane - kTopsPub] = sv;
     }
     if (lane == kTops - 1) sh.wtop[wave] = sv;
@@ -1206,13 +1207,14 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     slot_b = n_a + (uint32_t)__builtin_amdgcn_readfirstlane((int)wbase) + ((incl - mine) >> 16);
   }
   unsigned long long* out = a.cand + ((size_t)b * a.nchunks + c) * kCandCap;
+  const uint32_t cap = topk_more_tops(a.nchunks, rp.k) ? kCandCap - kMoreTops : kCandCap;  // entries of the list
   const bool restage = nst > (uint32_t)kScanStage;
 #pragma unroll
   for (int n = 0; n < kScanStage; ++n) {
     if (!restage && (uint32_t)n < nst) {  // the staged entries (the lane's own LDS column)
       const bool ta = (st_a >> n) & 1u;
       const uint32_t slot = ta ? slot_a : slot_b;
-      if (slot < (uint32_t)kCandCap) out[slot] = sh.stage[n][threadIdx.x];
+      if (slot < cap) out[slot] = sh.stage[n][threadIdx.x];
       slot_a += ta ? 1u : 0u;
       slot_b += ta ? 0u : 1u;
     }
@@ -1227,7 +1229,7 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
       if (l >= lo) {
         const bool ta = l >= th_a;
         const uint32_t slot = ta ? slot_a : slot_b;
-        if (slot < (uint32_t)kCandCap)
+        if (slot < cap)
           out[slot] = ((unsigned long long)radix_key(l / rp.tp) << 32) | (uint32_t)elem_index<VEC>(base, q * VEC + e);
         slot_a += ta ? 1u : 0u;
         slot_b += ta ? 0u : 1u;
@@ -1241,8 +1243,8 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     if (done == kThreads / 64 - 1) {
       const uint32_t n_a = atomicAdd(&sh.cnt, 0u), n = n_a + atomicAdd(&sh.cnt_b, 0u);
       a.cand_floor[(size_t)b * a.nchunks + c] = theta_v;
-      a.cand_count[(size_t)b * a.nchunks + c] = n > (uint32_t)kCandCap ? kCandCap + 1 : n;
-      a.cand_count_a[(size_t)b * a.nchunks + c] = n_a;
+      a.cand_count[(size_t)b * a.nchunks + c] = n > cap ? kCandCap + 1 : n;
+      a.cand_count_a[(size_t)b * a.nchunks + c] = n_a > cap ? kCandCap + 1 : n_a;
       a.cand_floor_a[(size_t)b * a.nchunks + c] = th_a;
     }
   }
@@ -1488,7 +1490,7 @@ __global__ void __launch_bounds__(kThreads) topk_select_kernel(SampleArgs a, flo
   const int b = blockIdx.x, K = a.topk, NC = a.nchunks;
   const char* row = row_ptr(a, b);
   TopkPrefetch pf;
-  topk_prefetch(a, b, pf);
+  topk_prefetch(a, b, K, pf);
   // the row's maximum key tells whether it holds a NaN
   unsigned long long mk = 0;
   for (int c = threadIdx.x; c < NC; c += blockDim.x) mk = max_u64(mk, a.chunk_max[(size_t)b * NC + c]);
@@ -1793,7 +1795,7 @@ __global__ void __launch_bounds__(kThreads) sample_select_kernel(SampleArgs a) {
   // chain of dependent steps); unused words are ignored
   const TfKey key = tf_key(a.keys[2 * b], a.keys[2 * b + 1]);
   TopkPrefetch pf;
-  topk_prefetch(a, b, pf);
+  topk_prefetch(a, b, rp.k, pf);
   unsigned long long mk = 0;
   for (int c = threadIdx.x; c < NC; c += blockDim.x) {
     const unsigned long long ck = a.chunk_max[(size_t)b * NC + c];
@@ -2371,6 +2373,7 @@ static SampleArgs make_args(const void* logits, int dtype, int batch, int vocab,
   const bool vec_ok = (vocab % vec) == 0 && (row_stride % vec) == 0 && (((uintptr_t)logits) & 15) == 0;
   a.chunk = kThreads * ((dtype != NVJSEL_F32 && vec_ok) ? 64 : 32);
   a.nchunks = (vocab + a.chunk - 1) / a.chunk;
+  a.last_fill = ((vocab - (a.nchunks - 1) * a.chunk) * 8 + a.chunk - 1) / a.chunk;
 
   a.stride = row_stride;
   a.lane_tops = (float*)(ws + w.lane_tops);
