@@ -527,10 +527,13 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
     }
     if constexpr (MODE == MODE_LOGITS) {
       // operands swapped: D[batch 8 (e >> 2) + 4 h + (e & 3)][vocab c32], so
-      // 32 lanes hold 32 consecutive logits of one row.  16-bit logits at
-      // addresses that allow it are transposed in quads of lanes (four rows x
-      // four columns) and stored 8 bytes per lane.
-      const bool quads = a.out_dtype != DT_F32 && ((a.V | (int)a.out_stride) & 3) == 0 && (((uintptr_t)a.out_logits) & 7) == 0;
+      // 32 lanes hold 32 consecutive logits of one row.  16-bit logits are
+      // transposed in quads of lanes (four rows x four columns) and stored 8
+      // bytes per lane, at any element address (V = 50,257, H = 512, B = 129 /
+      // 256 28 / 34 us, as 2-byte stores 42 / 52); the vocabulary's last quad may be partial.
+      typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+      typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
+      const bool quads = a.out_dtype != DT_F32;
 #pragma unroll
       for (int tv = 0; tv < TV; ++tv) {
         const int v = v0 + tv * 32 + c32;
@@ -544,8 +547,17 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
             for (int j = 0; j < 4; ++j) x[j] = apply_cast(acc[tv][tb][4 * i + j], a.reduce_cast);
             if (quads) {
               const uint2 q = quad_transpose16(x, a.out_dtype, lane);
-              if (v < vend && b + (lane & 3) < B)  // (vend is a multiple of 4: whole quads)
-                *(uint2*)((uint16_t*)a.out_logits + (size_t)(b + (lane & 3)) * (size_t)a.out_stride + (v & ~3)) = q;
+              const int left = vend - (v & ~3);  // columns of this quad
+              if (left > 0 && b + (lane & 3) < B) {
+                uint16_t* out = (uint16_t*)a.out_logits + (size_t)(b + (lane & 3)) * (size_t)a.out_stride + (v & ~3);
+                if (left >= 4) {
+                  *(u32x2_any_t*)out = u32x2_t{q.x, q.y};
+                } else {
+                  out[0] = (uint16_t)q.x;
+                  if (left > 1) out[1] = (uint16_t)(q.x >> 16);
+                  if (left > 2) out[2] = (uint16_t)q.y;
+                }
+              }
             } else {
 #pragma unroll
               for (int j = 0; j < 4; ++j)
