@@ -1386,8 +1386,14 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // Its 512-column strips leave CUs idle on a small vocabulary (V = 50,257, H
   // = 768, 99 blocks: sampled B = 1 / 4 / 8 30 / 36 / 46 us; the GEMM's 197
   // tiles ~28 at 1-16 rows), and f16 weights have no two-product dot there
-  // (V = 128,256, H = 2048, B = 1 / 8 84 / 142 us against 94)
-  const int hv_gemm_min = (V + 511) / 512 <= device_cu_count() / 2 ? 0
+  // (V = 128,256, H = 2048, B = 1 / 8 84 / 142 us against 94).  Rows of whole
+  // aligned groups stream faster: one row (V = 32,000, H = 512 / 1024 sampled 17
+  // / 27 us against 22 / 30), sampled two, four on short rows (H = 512, B = 2 / 4
+  // / 5 19 / 22 / 28 us against 22 / 24 / 24; H = 1024, B = 3 / 5 34 / 43 against
+  // 31 / 32)
+  const bool hv_vec8 = weight_dtype == NVJSEL_BF16 && aligned && (V % 8) == 0;
+  const int hv_gemm_min = (V + 511) / 512 <= device_cu_count() / 2
+                              ? (!hv_vec8 ? 0 : mode != MODE_SAMPLE ? 1 : H < 768 ? 4 : 2)
                           : weight_dtype == NVJSEL_F16             ? 2
                           : mode == MODE_SAMPLE                    ? kGemmHvMinBatchSample
                                                                    : kGemmHvMinBatch;
