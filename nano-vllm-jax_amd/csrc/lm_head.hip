@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "lm_head_common.h"
+#include "route_rules.h"
 
 // Launch shapes (chosen by measurement on MI355X).
 static constexpr int kLmWaves = 8;  // waves per block
@@ -971,19 +972,13 @@ static int launch_tile(const LmArgs& a, hipStream_t stream) {
   // a second epilogue wave per batch tile (sample mode; measured B=32 91 ->
   // 81 us, B=64 125 -> 118 us): two waves per SIMD issue the draws
   constexpr int EPM = (MODE == MODE_SAMPLE && NB >= 2) ? 2 : 1;
-  // (bf16 activations without sampling come here only for the fused prologue
-  // of up to kTilePrenormRows rows)
-  constexpr bool kPlain = NS == 3 || MODE == MODE_SAMPLE;
+  // (the fused prologue of bf16 activations: up to kTilePrenormRows rows)
   constexpr bool kFused = MODE != MODE_LOGITS && (NS == 3 || NB <= 2);
-  static_assert(kPlain || kFused, "some kernel serves the call");
-  if (a.prenorm ? !kFused : !kPlain) return fail(NVJSEL_EINVAL, "launch_tile: no such variant");
-  auto kern = [&]() {
-    if constexpr (kPlain && kFused)
-      return a.prenorm ? lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, true, NS>
-                       : lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, false, NS>;
-    else
-      return lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, kFused, NS>;
-  }();
+  auto kern = lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, false, NS>;
+  if (a.prenorm) {
+    if constexpr (kFused) kern = lm_head_tile_kernel<NB, GW, MODE, kTileDepth, EPM, true, NS>;
+    else return fail(NVJSEL_EINVAL, "launch_tile: no such variant");
+  }
   int grid = kTileBpc * device_cu_count();
   const int ntiles = (a.V + 15) / 16;
   if (grid > ntiles) grid = ntiles;
@@ -998,13 +993,9 @@ static int launch_tile(const LmArgs& a, hipStream_t stream) {
 template <int MODE>
 static int dispatch_tile(const LmArgs& a, hipStream_t s) {
   if (a.act_dtype != DT_BF16) return launch_tile<1, kTileW1, MODE, 3>(a, s);
-  if constexpr (MODE == MODE_LOGITS) return fail(NVJSEL_EINVAL, "dispatch_tile: bf16 logits take the staged GEMM");
-  else {
-    if (a.B <= 16) return launch_tile<1, kTileW1, MODE, 1>(a, s);
-    if (MODE != MODE_SAMPLE || a.B <= 32) return launch_tile<2, kTileW2, MODE, 1>(a, s);
-    if constexpr (MODE == MODE_SAMPLE) return launch_tile<4, kTileW4, MODE, 1>(a, s);
-  }
-  return NVJSEL_EINVAL;
+  if (a.B <= 16) return launch_tile<1, kTileW1, MODE, 1>(a, s);
+  if (a.B <= 32) return launch_tile<2, kTileW2, MODE, 1>(a, s);
+  return launch_tile<4, kTileW4, MODE, 1>(a, s);
 }
 
 // ------------------------------------------------------------------ generic kernel
@@ -1342,24 +1333,29 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   }
   // Staged GEMM on direct LDS loads (lm_head_ring.hip; 16-bit weight and
   // activations of one type).  Greedy and logits above the GEMV's rows: H =
-  // 1024, V = 248k, B = 16 / 64 / 100 / 256 76 / 78 / 88 / 136 us against 78 /
-  // 81 / 158 / 177 in 64-row tile passes and the blocked GEMM; logits B = 64 /
-  // 80 / 256 99 / 114 / 184 against 149 / 240 / 273; H = 2560, V = 152k, B =
+  // 1024, V = 248k, B = 16 / 64 / 100 / 256 76 / 78 / 84 / 131 us against 77 /
+  // 78 / 157 / 189 in 64-row tile passes and the blocked GEMM; logits B = 64 /
+  // 80 / 256 97 / 110 / 179 against 148 / 246 / 289; H = 2560, V = 152k, B =
   // 16 / 64 120 / 134 against 259 / 1010 in the straight-to-registers kernel.
-  // With the norm in the call (a prologue and a zeroing launch, ~11 us) the
-  // tile kernel's fused prologue stays up to 32 rows (85-88 us; 64 rows 100
-  // against 89).  Sampling: wherever the tile kernel does not take the shape,
-  // up to 128 rows per pass; where it does at 65-128 rows (B = 80 / 128 156 /
-  // 183 us against 177-185 / 202-209 in tile passes; B = 64 117-123 against
+  // Where the tile kernel takes the shape too, up to 64 rows by the share of W
+  // per block (ring_takes_small).  With the norm in the call (a prologue and a
+  // zeroing launch, ~11 us) the tile kernel's fused prologue stays up to 32
+  // rows (85-88 us; 64 rows 100 against 89).  Sampling: wherever the tile
+  // kernel does not take the shape, up to 128 rows per pass; where it does at
+  // 65-128 rows by the share (ring_takes_sample; B = 64 117-123 us against
   // 103-106) -- above 128 rows the blocked GEMM's single pass is faster (B =
   // 144 / 256 264 / 340 against 278 / 377), but for the band it leaves.
   const bool ring_ok = layout == NVJSEL_W_VH && aligned && weight_dtype != NVJSEL_F32 && eff_dtype == weight_dtype &&
                        (H % 64) == 0 && (prenorm || (((uintptr_t)hidden) & 15) == 0) &&
                        (mode != MODE_SAMPLE || V < (1 << 25));
   const bool ring1 = !gemv && ring_ok &&
-                    (mode != MODE_SAMPLE ? !(prenorm && tile_shape && batch <= kTilePrenormRows)
-                     : tile_shape        ? batch > 64 && batch <= kRingSampleRows
-                                         : batch <= kRingSampleRows || weight_dtype == NVJSEL_F16);
+                    (mode == MODE_SAMPLE
+                         ? (tile_shape ? batch > 64 && batch <= kRingSampleRows &&
+                                             ring_takes_sample(batch, V, device_cu_count())
+                                       : batch <= kRingSampleRows || weight_dtype == NVJSEL_F16)
+                         : !tile_shape || batch > 64 ||
+                               (!(prenorm && batch <= kTilePrenormRows) &&
+                                ring_takes_small(mode == MODE_LOGITS, batch, V, device_cu_count())));
   // f32 activations on bf16 [V, H] weights: the same kernel on three bf16
   // terms per value, 64 rows per pass (H = 1024, V = 248k, one box: greedy B =
   // 32 / 64 / 80 / 128 87 / 121 / 203 / 238 us, where 16-row tile passes and

@@ -42,6 +42,7 @@
 #include <limits.h>
 
 #include "lm_head_common.h"
+#include "route_rules.h"
 
 namespace nvjsel {
 
@@ -697,8 +698,7 @@ __global__ void __launch_bounds__(512) lm_head_ring_kernel(LmArgs a, int rows) {
 template <int WT, int MODE, int NBR, int NS>
 static int launch_ring_rows(const LmArgs& a, hipStream_t stream) {
   using S = RingShape<MODE, NBR, NS>;
-  const int cus = device_cu_count();
-  const int rows = ((a.V + cus - 1) / cus + 7) / 8 * 8;  // every block reads the same share of W, contiguous
+  const int rows = ring_share(a.V, device_cu_count());  // every block reads the same share of W, contiguous
   hipLaunchKernelGGL((lm_head_ring_kernel<WT, MODE, NBR, NS>), dim3((a.V + rows - 1) / rows), dim3(S::NW * 64), 0, stream,
                      a, rows);
   NVJSEL_CHECK_LAUNCH("lm_head_ring_kernel");

@@ -32,4 +32,48 @@ constexpr bool topk_tier_b(int nc, int k, int fill) {
   return 200 * e >= 73 * k && 1600 * nc <= 82 * k;
 }
 
+// ---- the staged GEMM (lm_head_ring.hip) against the tile kernel: 16-bit
+// weights [V, 1024] and bf16 activations, which both take.
+
+// Vocabulary rows per block of the staged GEMM, and the tiles of 256 they are
+// cut into: a remainder costs a whole tile's requests and products.
+constexpr int ring_share(int V, int cus) { return ((V + cus - 1) / cus + 7) / 8 * 8; }
+constexpr int ring_tiles(int share) { return (share + 255) / 256; }
+
+// Whether the staged GEMM takes a greedy / logits call of up to 64 rows.
+// Greedy: both stream W; the tile kernel (tiles of 16 rows, round robin) is
+// 2-30% faster on most vocabularies (V = 66,000 / 151,936 / 200,064, B = 16 24 /
+// 49 / 62 us against 31 / 52 / 68), equal on long shares that fill their tiles
+// (V = 248,320 / 311,296 76-77 / 95 both ways; not at whole MBs of W, 80 against
+// 84 at V = 262,144), and 3-12% slower from 49 rows on one well filled tile (V
+// = 57,344, B = 64 28.0 against 25.1).  Logits: the tile kernel stores a row's
+// logits 32 bytes at a time, so the staged GEMM is ahead from fewer full tiles
+// the more rows there are (V = 98,304, B = 8 / 16 / 24 / 64 34 / 36 / 40 / 59 us
+// in the tile kernel against 35 / 35 / 36 / 42).
+constexpr bool ring_takes_small(bool logits, int batch, int V, int cus) {
+  const int share = ring_share(V, cus), tiles = ring_tiles(share), full = 256 * tiles;
+  const bool longer = tiles >= 4 && 18 * share >= 17 * full && share % 1024 != 0;
+  if (!logits) return longer || (batch > 48 && tiles == 1 && 4 * share >= 3 * full);
+  if (batch <= 8) return longer;
+  if (batch <= 16) return 32 * share >= (batch <= 12 ? 28 : 25) * full && share != 256;
+  if (batch <= 24) return 4 * share >= 3 * full;
+  if (tiles == 1) return 8 * share >= 3 * full;
+  return batch > 32 || 8 * share >= 5 * full;
+}
+
+// Whether it takes a sampled call of 65-128 rows: it costs about 21 + 33 t, 13 +
+// 40 t, 13 + 41 t or 16 + 49 t us for t tiles (a remainder of a few rows half a
+// tile) at 65-68, 69-80, 81-96 or more rows, the tile kernel's two passes 22 +
+// 0.17 r, 24 + 0.18 r, 28 + 0.16 r or 30 + 0.18 r for a share of r rows (V = 98,304 / 248,320, B = 80 91 / 195 us in the tile kernel
+// against 92 / 166; B = 96 85 / 183 against 94 / 177; B = 128 95 / 201 against
+// 114 / 201).
+constexpr bool ring_takes_sample(int batch, int V, int cus) {
+  const int share = ring_share(V, cus), rem = share % 256;
+  const int t8 = share / 256 * 8 + (rem == 0 ? 0 : rem <= 16 ? 4 : rem <= 32 ? 5 : 8);  // eighths of tiles
+  if (batch <= 68) return 8 * share >= 205 * t8;
+  if (batch <= 80) return 8 * share >= 225 * t8 - 480;
+  if (batch <= 96) return 8 * share >= 255 * t8 - 744;
+  return 8 * share >= 270 * t8 - 480;
+}
+
 }  // namespace nvjsel
