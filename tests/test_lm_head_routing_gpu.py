@@ -1,15 +1,23 @@
 """GPU: every LM-head route at the batch sizes on both sides of its
 thresholds, against the oracle.
 
-The library picks among the streaming GEMV (greedy / logits up to 2 rows, 4
-for fp32 activations; sampling one fp32 row), the [H, V] streaming kernel, the
-MFMA tile kernel (64-row passes for bf16, 16-row for three-term fp32
-activations), the blocked GEMM (the kernel that idles padding waves below
-193 rows, the full-batch kernel above, 256-row passes beyond 256) and the
-three-term blocked GEMM (for fp32 activations at 65-128 rows: 64-row passes
-of its narrow layout while more rows are left than its threshold, then
-[V, H] 16-row tile passes and the GEMV for a rest of one or two rows, [H, V]
-8-row streaming passes), by layout, activation dtype, mode and batch.  Each
+[V, H] weights.  Streaming GEMV: greedy / logits up to 2 rows, 4 for fp32
+activations; sampling one fp32 row.  bf16 activations: the MFMA tile kernel up
+to 64 rows, and sampling in 64-row passes up to 128 (where the blocks' shares
+of W fill the staged GEMM's tiles, that one takes such calls: test_share_routes);
+the staged GEMM for greedy above 64 rows, 256 per pass; the blocked GEMM for
+sampling above 128, 256 per pass, but for 161-192 rows (tile passes).  fp32
+activations: 16-row passes of the tile kernel up to 16 rows, the staged GEMM on
+three terms in 64-row passes up to 192 (a rest of at most 16 rows in the tile
+kernel, of one or two in the GEMV), the blocked GEMM above, 256 per pass.
+
+[H, V] weights.  On this vocabulary (few 512-column strips) the blocked GEMM
+takes bf16 activations from 2 rows (sampled 3), the streaming kernel fewer; its
+narrow layout up to 64 rows, the one that idles padding waves up to 192.  fp32
+activations: streaming up to 8 rows, the blocked GEMM above; at 65-128 rows
+64-row passes of its narrow layout, then 8-row streaming passes.
+
+Each
 case checks greedy ids (check_greedy: first index of the maximum of the
 rounded logits, rows within the fp32-summation flip accepted) or sampled ids
 (check_fused_sampled: the oracle's Gumbel-max scores) on a vocabulary that is
@@ -75,3 +83,31 @@ def test_sample_routes(weights, layout, act, B):
     # 66, bf16: 5 such rows, the same ids from the [V, H] tile passes and the
     # [H, V] blocked GEMM)
     assert namb <= max(2, B // 8)
+
+
+@pytest.mark.parametrize("mode,B", [("greedy", 16), ("greedy", 49), ("logits", 8), ("logits", 9), ("logits", 40),
+                                    ("sample", 65), ("sample", 97)])
+def test_share_routes(mode, B):
+    """bf16 calls that the tile kernel and the staged GEMM both take, on a
+    vocabulary whose shares fill the staged GEMM's tiles on 256 CUs (248 of 256
+    rows): greedy above 48 rows, logits above 8 and sampled above 64 go there."""
+    v = 62470
+    rng = np.random.default_rng(B)
+    h = bf16_tensor(rng.standard_normal((B, H)))
+    w = bf16_tensor(rng.standard_normal((v, H)) * 0.05)
+    z = sel.lm_head_logits(h.float().cpu().numpy(), w.float().cpu().numpy())
+    ctx = f"share route {mode} B={B}"
+    if mode == "sample":
+        T = [float(x) for x in rng.choice([0.0, 0.8, 1.0], B)]
+        keys = engine_keys(B, 11)
+        ids = nvjsel.lm_head_sample_token_ids(h, w, temperatures=torch.tensor(T).cuda(), rng_keys=keys_tensor(keys),
+                                              weight_layout="vh")
+        assert check_fused_sampled(ids.cpu().numpy(), z, T, keys, 1, ctx) <= B // 8
+    elif mode == "greedy":
+        check_greedy(nvjsel.lm_head_greedy_top1_hip(h, w, weight_layout="vh").cpu().numpy(), z, 1, ctx)
+    else:
+        got = nvjsel.lm_head_logits_hip(h, w, weight_layout="vh").float().cpu().numpy().astype(np.float64)
+        # fp32 sums of H products and one rounding to bf16
+        hn = np.linalg.norm(h.float().cpu().numpy(), axis=1)[:, None]
+        wn = np.linalg.norm(w.float().cpu().numpy(), axis=1)[None, :]
+        assert (np.abs(got - z) <= H * 2.0 ** -23 * hn * wn + np.abs(z) * 2.0 ** -8 + 1e-7).all()

@@ -33,9 +33,9 @@ def _inputs(rng, batch, H, V, hidden_dtype):
     (2, 1024, "f32", "f32"),     # streaming GEMV, fused, fp32 operand
     (1, 512, "bf16", "f32"),     # streaming GEMV, fused, H = 512
     (5, 1024, "bf16", "bf16"),   # tile kernel, fused
-    (64, 1024, "f32", "bf16"),   # tile kernel, fused, f32 input
-    (70, 1024, "bf16", "bf16"),  # blocked GEMM, prologue kernel
-    (82, 1024, "bf16", "f32"),   # fp32 operand, 65-128 rows: narrow GEMM + tile pass + GEMV, prologue kernel
+    (64, 1024, "f32", "bf16"),   # tile kernel, f32 input, prologue kernel
+    (70, 1024, "bf16", "bf16"),  # staged GEMM, prologue kernel
+    (82, 1024, "bf16", "f32"),   # fp32 operand: 64 rows in the staged GEMM, 16 in the tile kernel, 2 in the GEMV
     (8, 1024, "bf16", "f32"),    # exact-split MFMA path, prologue kernel
     (4, 40, "f16", "f32"),       # generic path, prologue kernel
 ])
