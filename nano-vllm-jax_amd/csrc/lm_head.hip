@@ -1382,14 +1382,18 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // Its 512-column strips leave CUs idle on a small vocabulary (V = 50,257, H
   // = 768, 99 blocks: sampled B = 1 / 4 / 8 30 / 36 / 46 us; the GEMM's 197
   // tiles ~28 at 1-16 rows), and f16 weights have no two-product dot there
-  // (V = 128,256, H = 2048, B = 1 / 8 84 / 142 us against 94).  Rows of whole
-  // aligned groups stream faster: one row (V = 32,000, H = 512 / 1024 sampled 17
-  // / 27 us against 22 / 30), sampled two, four on short rows (H = 512, B = 2 / 4
-  // / 5 19 / 22 / 28 us against 22 / 24 / 24; H = 1024, B = 3 / 5 34 / 43 against
-  // 31 / 32)
+  // (V = 128,256, H = 2048, B = 1 / 8 84 / 142 us against 94).  Whole aligned
+  // groups of short weights stream faster: greedy / logits of one row at H < 1024
+  // (V = 32,000, H = 512 15.9 us against 16.5; H = 1024 26.4 against 23.4),
+  // sampled of one row at H < 2048 (H = 1024 / 2048 27.5 / 46 against 30.3 / 44),
+  // two at H < 1024 (H = 768 / 1024, B = 2 23.8 / 30.3 against 26.4 / 30.3), four
+  // at H < 768 (H = 512, B = 4 / 5 22.4 / 28.3 against 23.7 / 23.6; H = 768, B = 3
+  // 27.8 against 26.6)
   const bool hv_vec8 = weight_dtype == NVJSEL_BF16 && aligned && (V % 8) == 0;
-  const int hv_gemm_min = (V + 511) / 512 <= device_cu_count() / 2
-                              ? (!hv_vec8 ? 0 : mode != MODE_SAMPLE ? 1 : H < 768 ? 4 : 2)
+  const int hv_small_min = !hv_vec8              ? 0
+                           : mode != MODE_SAMPLE ? (H < 1024 ? 1 : 0)
+                                                 : (H < 768 ? 4 : H < 1024 ? 2 : H < 2048 ? 1 : 0);
+  const int hv_gemm_min = (V + 511) / 512 <= device_cu_count() / 2 ? hv_small_min
                           : weight_dtype == NVJSEL_F16             ? 2
                           : mode == MODE_SAMPLE                    ? kGemmHvMinBatchSample
                                                                    : kGemmHvMinBatch;
