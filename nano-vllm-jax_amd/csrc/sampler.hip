@@ -641,7 +641,7 @@ struct TopkPrefetch {
   unsigned long long cv[4];  // entries (t & 7) + 8 q of chunk t >> 3's list (the gather's first reads)
 };
 
-__device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, int k, TopkPrefetch& pf) {
+__device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPrefetch& pf) {
   const int NC = a.nchunks;
   pf.cnt = 0;
   pf.cnt_a = 0;
@@ -668,14 +668,19 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, int k,
   const unsigned long long* src = a.cand + ((size_t)b * NC + (c < NC ? c : 0)) * kCandCap;
 #pragma unroll
   for (int q = 0; q < 4; ++q) pf.cv[q] = src[(threadIdx.x & 7) + 8 * q];
-  // last, and only for rows that want them: read for every row (so that they
-  // need not wait for k) they cost k = 20 rows 0.3 us
-  if (topk_more_tops(NC, k)) {
+}
+
+// The second four's, for rows that want them (topk_more_tops): requested once k
+// is here and the chunk maxima are on their way, before those are reduced (for
+// every row in topk_prefetch, or there once k had come, k = 20 rows took 0.3-0.5
+// us longer).
+__device__ __forceinline__ void topk_prefetch_more(const SampleArgs& a, int b, int k, TopkPrefetch& pf) {
+  const int NC = a.nchunks;
+  if (!topk_more_tops(NC, k)) return;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {  // (key[2] and [3] are free: k <= 256, so 16 NC <= 352; other rows drop them)
-      const int j = (int)threadIdx.x + kThreads * i;
-      if (j < NC * (kThreads / 64) * kTopsPub) pf.key[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
-    }
+  for (int i = 0; i < 2; ++i) {  // (k <= 256: 16 NC <= 352 values, so key[2] and [3] are free)
+    const int j = (int)threadIdx.x + kThreads * i;
+    if (j < NC * (kThreads / 64) * kTopsPub) pf.key[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
   }
 }
 
@@ -1490,10 +1495,11 @@ __global__ void __launch_bounds__(kThreads) topk_select_kernel(SampleArgs a, flo
   const int b = blockIdx.x, K = a.topk, NC = a.nchunks;
   const char* row = row_ptr(a, b);
   TopkPrefetch pf;
-  topk_prefetch(a, b, K, pf);
+  topk_prefetch(a, b, pf);
   // the row's maximum key tells whether it holds a NaN
   unsigned long long mk = 0;
   for (int c = threadIdx.x; c < NC; c += blockDim.x) mk = max_u64(mk, a.chunk_max[(size_t)b * NC + c]);
+  topk_prefetch_more(a, b, K, pf);
   mk = block_max_u64(mk, s.red);
   bool fast = (uint32_t)(mk >> 32) != 0xFFFFFFFFu;
   if (fast) {
@@ -1795,7 +1801,7 @@ __global__ void __launch_bounds__(kThreads) sample_select_kernel(SampleArgs a) {
   // chain of dependent steps); unused words are ignored
   const TfKey key = tf_key(a.keys[2 * b], a.keys[2 * b + 1]);
   TopkPrefetch pf;
-  topk_prefetch(a, b, rp.k, pf);
+  topk_prefetch(a, b, pf);
   unsigned long long mk = 0;
   for (int c = threadIdx.x; c < NC; c += blockDim.x) {
     const unsigned long long ck = a.chunk_max[(size_t)b * NC + c];
@@ -1822,6 +1828,7 @@ __global__ void __launch_bounds__(kThreads) sample_select_kernel(SampleArgs a) {
     return;
   }
   const bool fast_topk = rp.mode == ROW_FILTER && rp.k > 0 && rp.k <= kFastK;
+  if (fast_topk) topk_prefetch_more(a, b, rp.k, pf);
   const bool topp_only = rp.mode == ROW_FILTER && rp.k == 0 && rp.p < 1.0f;
   int tbm = INT_MIN;  // top-p-only rows: the chunks' top grid bins, loaded with the maxima
   if (topp_only)
