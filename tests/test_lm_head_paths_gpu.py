@@ -152,8 +152,8 @@ def test_fp32_activations_sample():
     assert check_fused_sampled(ids.cpu().numpy(), z, T, keys, 0, "f32 act sample") <= 1
 
 
-# (B, H, layout, act, weight dtype): streaming [V,H] B<=2, fp32 B<=8, tile 3..64 and
-# 64-row chunks, [H,V], f16 MFMA, generic (H not a multiple of 32)
+# (B, H, layout, act, weight dtype): streaming [V,H] B<=2, fp32 tile B<=16, tile or
+# staged GEMM above (fp32: three terms), [H,V], f16 staged, generic (H not a multiple of 32)
 LOGIT_CASES = [
     (1, 1024, "vh", torch.bfloat16, torch.bfloat16),
     (2, 512, "vh", torch.float32, torch.bfloat16),
@@ -250,12 +250,11 @@ def test_gemm_greedy_and_logits(B, H):
 @pytest.mark.parametrize("B,H", [(33, 1024), (64, 1024), (65, 512), (81, 1024), (100, 1024), (200, 1024),
                                  (300, 1024), (32, 1024)])
 def test_gemm_f32_activations(B, H):
-    """fp32 activations (lm_head_decode_act_dtype fp32) above 32 rows: the
-    blocked GEMM on three bf16 terms per value (the narrow layout up to 64
-    rows; at H = 1024 and 65-128 rows 64-row narrow passes, then 16-row tile
-    passes and the GEMV for a last row: B = 81, 100) -- one pass over W per
-    256 rows, greedy and logits -- against the float64 dot (fp32 logits); 32
-    rows take two 16-row tile passes."""
+    """fp32 activations (lm_head_decode_act_dtype fp32) above 16 rows on three
+    bf16 terms per value: 64-row passes of the staged GEMM up to 192 rows left
+    (at H = 1024 a rest of up to 16 rows in the tile kernel, of one or two in
+    the GEMV: B = 81), 256-row passes of the blocked GEMM above (B = 200, 300),
+    greedy and logits, against the float64 dot (fp32 logits)."""
     rng = np.random.default_rng(7700 + B + H)
     V = 9001
     W = bf16_tensor(rng.standard_normal((V, H)) * 0.05)
@@ -271,11 +270,11 @@ def test_gemm_f32_activations(B, H):
 
 @pytest.mark.parametrize("B", [33, 60, 85, 300])
 def test_gemm_sample_f32_activations(B):
-    """Fused Gumbel sampling with fp32 activations at 33-64 rows (the narrow
-    layout, 32-wide K stages) and above 80 rows (the full layout, 16-wide K
-    stages; B = 300: two 256-row passes) -- the blocked GEMM on three bf16
-    terms -- greedy rows beside temperature rows, against the oracle's scores
-    on the float64 logits (fp32 logits, no rounding)."""
+    """Fused Gumbel sampling with fp32 activations on three bf16 terms: 64-row
+    passes of the staged GEMM up to 192 rows, the blocked GEMM's 256 above
+    (16-wide K stages; B = 300: 256 rows, then 44) -- greedy rows beside
+    temperature rows, against the oracle's scores on the float64 logits (fp32
+    logits, no rounding)."""
     rng = np.random.default_rng(9300 + B)
     H, V = 1024, 12007
     W = bf16_tensor(rng.standard_normal((V, H)) * 0.05)
@@ -348,10 +347,11 @@ def test_gemm_hv_greedy_winner_in_last_columns():
 
 @pytest.mark.parametrize("B,act", [(130, torch.bfloat16), (100, torch.float32)])
 def test_gemm_hv_matches_vh_bitwise(B, act):
-    """Where both layouts run the blocked GEMM (bf16 above 64 rows; fp32
-    activations at 100 rows: two narrow passes on either layout), the [H, V] kernel multiplies the same products
-    in the same k order as the [V, H] one: logits bitwise equal, sampled ids
-    equal."""
+    """bf16 at 130 rows (logits and greedy [V, H] in the staged GEMM, the rest
+    in the blocked one) and fp32 activations at 100 (64-row passes of the staged
+    GEMM, narrow passes of the blocked one): the kernels multiply the same
+    products in the same k order on either layout: logits bitwise equal, sampled
+    ids equal."""
     rng = np.random.default_rng(9600 + B)
     H, V = 1024, 12008
     Wvh = bf16_tensor(rng.standard_normal((V, H)) * 0.05)
@@ -395,15 +395,18 @@ def test_gemm_hv_sample(B, act):
 
 
 @pytest.mark.parametrize("rc", [0, 2])
-def test_gemm_other_roundings(rc):
-    """The blocked GEMM with the caller's reduce_cast: 0 (fp32 logits, f32
-    out) and 2 (f16 rounding), greedy and logits."""
+@pytest.mark.parametrize("layout", ["vh", "hv"])
+def test_gemm_other_roundings(layout, rc):
+    """The staged ([V, H]) and the blocked GEMM ([H, V]) with the caller's
+    reduce_cast: 0 (fp32 logits, f32 out) and 2 (f16 rounding), greedy and
+    logits."""
     rng = np.random.default_rng(880 + rc)
     B, H, V = 96, 512, 7001
     W = bf16_tensor(rng.standard_normal((V, H)) * 0.05)
     h = _hidden(rng, B, H, torch.bfloat16)
-    ids = nvjsel.lm_head_greedy_top1_hip(h, W.T, reduce_cast=rc)
-    logits = nvjsel.lm_head_logits_hip(h, W.T, reduce_cast=rc)
+    wo = W if layout == "vh" else W.T.contiguous()
+    ids = nvjsel.lm_head_greedy_top1_hip(h, wo, weight_layout=layout, reduce_cast=rc)
+    logits = nvjsel.lm_head_logits_hip(h, wo, weight_layout=layout, reduce_cast=rc)
     torch.cuda.synchronize()
     hf, wf = h.float().cpu().numpy(), W.float().cpu().numpy()
     check_greedy(ids.cpu().numpy().reshape(-1), sel.lm_head_logits(hf, wf), rc, f"gemm rc={rc}")
@@ -429,10 +432,10 @@ def test_gemm_full_vocab_b256_with_prenorm():
 
 @pytest.mark.parametrize("B,H", [(65, 512), (130, 1024), (200, 1024), (256, 1024), (300, 1024), (513, 512)])
 def test_gemm_sample_mixed_temperatures(B, H):
-    """Fused Gumbel sampling through the blocked GEMM (above 64 rows, above
-    192 where the tile kernel serves H = 1024: B = 130 takes 64-row tile
-    passes; B = 300 and 513 take two and three 256-row passes that reuse the
-    row keys and the ticket): greedy rows (T = 0) beside temperature rows, a
+    """Fused Gumbel sampling through the blocked GEMM above 128 rows (H = 1024:
+    B = 130, 256 and, 256-row passes that reuse the row keys and the ticket,
+    300; 200 too; H = 512: three passes of 513) and the staged one (B = 65, H =
+    512): greedy rows (T = 0) beside temperature rows, a
     vocabulary that is not a multiple of the 256-row tile, against the
     oracle's scores s_v = rnd(z_v)/T + g_v."""
     rng = np.random.default_rng(9100 + B + H)
@@ -497,11 +500,14 @@ def test_gemm_sample_bench_workload_b256():
 
 
 @pytest.mark.parametrize("rc", [0, 2])
-def test_gemm_sample_other_roundings(rc):
-    """Sample mode of the blocked GEMM with fp32 (0) and f16 (2) rounding of
-    the logits before the draws, greedy rows beside temperature rows."""
+@pytest.mark.parametrize("B,H", [(100, 1024), (100, 512), (140, 1024)])
+def test_gemm_sample_other_roundings(B, H, rc):
+    """Sample mode of the tile kernel (100 rows at H = 1024, this vocabulary),
+    the staged (H = 512) and the blocked GEMM (140 rows) with fp32 (0) and f16
+    (2) rounding of the logits before the draws, greedy rows beside temperature
+    rows."""
     rng = np.random.default_rng(9500 + rc)
-    B, H, V = 100, 1024, 12007
+    V = 12007
     W = bf16_tensor(rng.standard_normal((V, H)) * 0.05)
     h = _hidden(rng, B, H, torch.bfloat16)
     T = [float(x) for x in rng.choice([0.0, 0.8, 1.0], B)]
