@@ -345,7 +345,7 @@ def build_configs(torch, which, with_cpu):
         desc = {"x3": "greedy LM-head top-1, B=1, W [1024,248320] bf16 ([H,V], the materialised lm_head)",
                 "x4": "greedy LM-head top-1, B=8, W [1024,248320] bf16 ([H,V])",
                 "x5": "greedy LM-head top-1, B=8, fp32 activations x W [248320,1024] bf16 (one W pass)",
-                "x6": "greedy LM-head top-1, B=256, bf16 x W [248320,1024] bf16 (one W pass, blocked GEMM)"}[name]
+                "x6": "greedy LM-head top-1, B=256, bf16 x W [248320,1024] bf16 (one W pass, staged GEMM)"}[name]
         kern = {"x5": "lm_head_tile_kernel", "x6": "lm_head_ring_kernel"}.get(name, "lm_head_hv_kernel")
         tag = "hv" if layout else {"x5": "f32act", "x6": "gemm"}[name]
         cfgs.append(Cfg(f"{name}_{tag}_greedy_b{B}", B,

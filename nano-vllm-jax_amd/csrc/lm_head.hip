@@ -1179,7 +1179,7 @@ static size_t lm_ws_small_bytes(int batch) {
 static constexpr int kGemmMinBatchTileSample = 192;
 static constexpr int kGemmBandSample = 160;
 static constexpr int kTilePrenormRows = 32;  // bf16 activations: the fused prologue of the tile kernel up to here
-// [H, V] weights: the GEMM above 8 rows for bf16 activations (V = 248k, up
+// [H, V] weights of many strips (hv_gemm_min): the GEMM above 8 rows for bf16 activations (V = 248k, up
 // to 64 rows in the narrow layout: ~94-98 us greedy, ~113-143 us sampled,
 // against 8-row streaming passes of ~88-100 us each) and for fp32 above 8
 // (~168-180 / ~185-218 us against passes of ~97 / ~111 us: B = 12 sampled
@@ -1373,8 +1373,8 @@ static int lm_head_entry(int mode, const void* hidden, int hidden_dtype, const v
   // blocked GEMM: sampling bf16 activations on [V, H] above 128 rows (H =
   // 1024: at 129-160 and above 192), one pass over W per 256 rows (sample
   // mode packs vocabulary ids into 25 bits of its queue entries); [H, V]
-  // weights (transposing LDS reads) from 9 rows, every mode; the [H, V]
-  // streaming kernel takes 8 rows per pass over W
+  // weights (transposing LDS reads) every mode, above the rows of the [H, V]
+  // streaming kernel, which takes 8 per pass over W (hv_gemm_min)
   const bool hv_gemm_ok = layout == NVJSEL_W_HV && V >= 8 && (((uintptr_t)weight) & 1) == 0 &&
                           (weight_dtype == NVJSEL_BF16 || (weight_dtype == NVJSEL_F16 && eff_dtype == NVJSEL_F16));
   const bool gemm_ok = (bf16_mfma || hv_gemm_ok) && (H % (2 * kGemmKC)) == 0 &&

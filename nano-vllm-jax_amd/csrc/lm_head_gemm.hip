@@ -1,15 +1,18 @@
 // LM head as a blocked GEMM staged through registers into the LDS (gfx950):
-// [H, V] weights from 9 rows (every mode); on [V, H] bf16 sampling above 128
-// rows and f32 activations above 192.
+// [H, V] weights, every mode, above the streaming kernel's rows (8; 16-bit
+// activations fewer on f16 weights and on vocabularies up to 512 columns for
+// half of the CUs, from the first row); on [V, H] bf16 sampling above 128 rows
+// and f32 activations above 192.
 #include "lm_head_common.h"
 
 namespace nvjsel {
 
-// ------------------------------------------------------------------ blocked GEMM, 64 < B <= 256
-// bf16 hidden x bf16 W [V, H], H % 64 == 0, up to 256 rows in ONE pass over
-// W.  The hidden of 256 rows (512 KB at H = 1024) is a CU's whole register
-// file, so unlike the tile kernel nothing is held for the whole call: a block
-// tile is 256 vocabulary rows x all 256 batch rows, and K is streamed in
+// ------------------------------------------------------------------ blocked GEMM, 1 <= B <= 256
+// 16-bit W [V, H] or [H, V], hidden of the same type or f32 on bf16, H % 64 ==
+// 0, up to 256 rows in ONE pass over W (f16: 64).  The hidden of 256 rows (512
+// KB at H = 1024) is a CU's whole register file, so unlike the tile kernel
+// nothing is held for the whole call: a block tile is 256 vocabulary rows x all
+// 256 batch rows (NARROW, 64 rows and fewer: below), and K is streamed in
 // stages of 32 -- the W stage (256 x 32, 16 KB, from HBM) and the hidden
 // stage (256 x 32, 16 KB, L2-resident) staged through a two-buffer LDS ring.
 // Each thread loads 4 x 16 B per stage into registers; two register sets
@@ -37,7 +40,7 @@ static constexpr int kGemmQcap = 768;  // queue entries per wave (sample mode; L
 // beats the lane's running best (bo, bi) is the first element rounding to it
 // looked up.  Rounding is monotone, so max(round(x)) = round(max(x)), and ties
 // keep the lowest vocabulary row (rows ascend with e and with the tiles).
-// Rows past V hold re-read data ([V, H]: row V - 1; [H, V]: the last 8-column
+// Rows past V hold other data ([V, H]: row V - 1; [H, V]: the last or the next row's
 // group) and are masked in the last tile.
 template <int MODE, int TV>
 __device__ __forceinline__ void gemm_epilogue(const LmArgs& a, const f32x16_t (&acc)[TV][2], int v0, int bj, int h,

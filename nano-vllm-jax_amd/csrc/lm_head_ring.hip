@@ -36,6 +36,10 @@
 //    B = 16 took 99 us against 87).  Fragment reads bound it at 64 rows: 64 x
 //    32 per wave instead of 32 x 64 reads 160 KB per stage instead of 224 (B =
 //    64 126 -> 121 us).
+//  * A share that ends in part of a tile pays the whole one's requests and
+//    products (V = 66,000, two tiles for 264 rows, B = 16 31 us where the tile
+//    kernel takes 24): bf16 calls at H = 1024 that the tile kernel takes too go by
+//    the share (route_rules.h).
 // H = 1024, V = 248,320, greedy B = 16 / 64 / 128 / 256: 76 / 78 / 90 / 136 us
 // (6.6 / 6.5 / 5.7 / 3.7 TB/s; 956 TFLOP/s at 256) where 64-row passes of the
 // tile kernel and the blocked GEMM took 78 / 81 / 160 / 177.
