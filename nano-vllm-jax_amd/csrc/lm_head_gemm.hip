@@ -135,9 +135,9 @@ __device__ __forceinline__ void gemm_finish_rows(const LmArgs& a, unsigned long 
 // one.  Else rows start at any element (V >= 8): 16-byte loads from element
 // addresses; a group that ends past its row reads on into the next one (columns
 // masked where they could win), in the last row it is loaded from V - 8 and
-// moved down as it is stored: 2-4% more time on aligned rows of f32 hidden (V =
-// 32,000, H = 1024, B = 32 48.8 us against 47.6; 16-bit hidden 24.1 with VEC8,
-// 23.2 without).
+// moved down as it is stored: 2-6% more time on aligned rows (V = 32,000, H =
+// 1024, f32 hidden B = 32 48.8 us against 47.6, bf16 B = 256 46.7 against 44.4),
+// but for 16-bit hidden in the narrow layout (B = 32 23.2 against 24.1 with VEC8).
 template <int WT, int MODE, int BV, int NS, int KC, bool HV, bool VEC8, bool PART, bool NARROW>
 __global__ void __launch_bounds__(BV * 2, 256 / BV) lm_head_gemm_kernel(LmArgs a) {
   constexpr int Q = KC / 8;  // 8-element columns per row and stage
@@ -551,7 +551,7 @@ static int launch_gemm_shape(const LmArgs& a, hipStream_t stream) {
   constexpr bool kNarrow = HV;
   if constexpr (kNarrow) {
     if (a.B <= 64) {
-      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, kGemmKC, HV, VEC8, false, true>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
+      hipLaunchKernelGGL((lm_head_gemm_kernel<WT, MODE, kGemmBV, NS, kGemmKC, HV, VEC8 && NS == 3, false, true>), dim3(grid), dim3(kGemmBV * 2), 0, stream, a);
       NVJSEL_CHECK_LAUNCH("lm_head_gemm_kernel");
       return NVJSEL_OK;
     }
@@ -588,14 +588,16 @@ int launch_gemm(int mode, bool hv, const LmArgs& a, hipStream_t stream) {
   // (f16 weights take the any-element loads: their rows were never faster)
   if (a.weight_dtype == DT_F16)
     return by_mode([&](auto M) { return launch_gemm_shape<DT_F16, decltype(M)::value, 1, true, false>(a, stream); });
-  if (a.hidden_dtype == DT_F32) {
-    const bool vec8 = (a.V % 8) == 0 && (((uintptr_t)a.W) & 15) == 0;
+  const bool vec8 = (a.V % 8) == 0 && (((uintptr_t)a.W) & 15) == 0;
+  if (a.hidden_dtype == DT_F32)
     return by_mode([&](auto M) {
       return vec8 ? launch_gemm_shape<DT_BF16, decltype(M)::value, 3, true, true>(a, stream)
                   : launch_gemm_shape<DT_BF16, decltype(M)::value, 3, true, false>(a, stream);
     });
-  }
-  return by_mode([&](auto M) { return launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true, false>(a, stream); });
+  return by_mode([&](auto M) {
+    return vec8 ? launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true, true>(a, stream)
+                : launch_gemm_shape<DT_BF16, decltype(M)::value, 1, true, false>(a, stream);
+  });
 }
 
 }  // namespace nvjsel
