@@ -11,8 +11,8 @@ namespace nvjsel {
 // the k-th of the 16 nc published values and the largest chunk floor -- reaches
 // every chunk's tier A, and takes a whole-row descent if not (64 f32 rows at 10
 // chunks 380 us against 25).  k <= 32 rows always settle (a chunk's own floor
-// does); the others want twice the published values until 16 nc = 7/5 k (one
-// more load: no measured cost), and below 16 nc = k tier B, the lists down to
+// does); the others take the next four of each wave too until 16 nc = 7/5 k (they
+// come in the same words), and below 16 nc = k tier B, the lists down to
 // the chunk's own floor (k = 128-160 rows 31 us with it where they settle
 // without, 26), as long as its floors come out high enough:
 //  * from the published values, once 32 nc (counting the last chunk's fill)

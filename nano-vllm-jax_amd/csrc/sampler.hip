@@ -110,7 +110,8 @@ struct SampleArgs {
   uint32_t* list_n;                // [2]   rows queued for gumbel, for top-p
   uint32_t* list_gumbel;           // [B * nchunks] gumbel items: row << 16 | chunk
   int32_t* out_ids;
-  float* lane_tops;                // [B, nchunks, 4 waves, kTopsPub] largest raw-logit lane maxima
+  uint32_t* lane_tops;             // [B, nchunks, 4 waves, kTopsPub] the 2 kTopsPub largest lane maxima of a wave
+                                   // (top halves of their radix keys): word t holds the t-th and the (t + 4)-th
   int topk;  // > 0: top-k selection (nvjsel_topk): every row FILTER with this k on raw logits
   // nvjsel_debug_sample_topp only (null otherwise): each FILTER row's final
   // threshold (x space) and the softmax mass of its kept set over the top-k
@@ -623,13 +624,6 @@ struct FinishShared {
 __device__ __forceinline__ bool scan_tier_b(const SampleArgs& a, const RowParams& rp) {
   return a.topk > 0 || topk_tier_b(a.nchunks, rp.k, a.last_fill);
 }
-// Chunk c's second four lane maxima per wave (16 floats): the last eight entries
-// of its list, whose page scan and select touch anyway.
-static constexpr int kMoreTops = 8;
-__device__ __forceinline__ float* more_tops(const SampleArgs& a, int b, int c) {
-  return (float*)(a.cand + ((size_t)b * a.nchunks + c) * kCandCap + (kCandCap - kMoreTops));
-}
-
 // The first loads of a fast top-k row, issued by select before it reduces the
 // chunk maxima so that both are in flight together: each chunk's tier A count
 // and floors (thread c), and the row's published lane maxima as 16-bit keys
@@ -637,7 +631,7 @@ __device__ __forceinline__ float* more_tops(const SampleArgs& a, int b, int c) {
 struct TopkPrefetch {
   uint32_t cnt, cnt_a;
   float fl_a, fl;
-  uint32_t key[4];  // published lane maxima t + 256 i, as 16-bit keys (0: none); [2], [3]: topk_more_tops
+  uint32_t tops[4];  // published words t + 256 i (0: none)
   unsigned long long cv[4];  // entries (t & 7) + 8 q of chunk t >> 3's list (the gather's first reads)
 };
 
@@ -655,11 +649,11 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPr
     pf.fl = a.cand_floor[i];
   }
   const int nvals = min(NC, kTopsChunks) * (kThreads / 64) * kTopsPub;
-  const float* tops = a.lane_tops + (size_t)b * NC * (kThreads / 64) * kTopsPub;
+  const uint32_t* tops = a.lane_tops + (size_t)b * NC * (kThreads / 64) * kTopsPub;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = (int)threadIdx.x + kThreads * i;
-    pf.key[i] = j < nvals ? radix_key(tops[j]) >> 16 : 0u;
+    pf.tops[i] = j < nvals ? tops[j] : 0u;
   }
   // the first list entries the gather reads, requested now rather than once
   // the row floor is known (inside each chunk's list area; entries past the
@@ -668,20 +662,6 @@ __device__ __forceinline__ void topk_prefetch(const SampleArgs& a, int b, TopkPr
   const unsigned long long* src = a.cand + ((size_t)b * NC + (c < NC ? c : 0)) * kCandCap;
 #pragma unroll
   for (int q = 0; q < 4; ++q) pf.cv[q] = src[(threadIdx.x & 7) + 8 * q];
-}
-
-// The second four's, for rows that want them (topk_more_tops): requested once k
-// is here and the chunk maxima are on their way, before those are reduced (for
-// every row in topk_prefetch, or there once k had come, k = 20 rows took 0.3-0.5
-// us longer).
-__device__ __forceinline__ void topk_prefetch_more(const SampleArgs& a, int b, int k, TopkPrefetch& pf) {
-  const int NC = a.nchunks;
-  if (!topk_more_tops(NC, k)) return;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {  // (k <= 256: 16 NC <= 352 values, so key[2] and [3] are free)
-    const int j = (int)threadIdx.x + kThreads * i;
-    if (j < NC * (kThreads / 64) * kTopsPub) pf.key[2 + i] = radix_key(more_tops(a, b, j >> 4)[j & 15]) >> 16;
-  }
 }
 
 // Largest 16-bit prefix p with at least k of the row's published lane maxima
@@ -729,7 +709,11 @@ __device__ int topk_sorted_survivors(const SampleArgs& a, int b, const RowParams
     s.cnt_a[threadIdx.x] = pf.cnt_a;
     s.fl_a[threadIdx.x] = pf.fl_a;
   }
-  const uint32_t kf16 = row_tops_kth(pf.key, rp.k, s) << 16;
+  // (topk_more_tops: at most 22 chunks, 352 words, all in tops[0] and [1])
+  const bool more = topk_more_tops(NC, rp.k);
+  const uint32_t keys[4] = {pf.tops[0] & 0xFFFFu, pf.tops[1] & 0xFFFFu, more ? pf.tops[0] >> 16 : pf.tops[2] & 0xFFFFu,
+                            more ? pf.tops[1] >> 16 : pf.tops[3] & 0xFFFFu};
+  const uint32_t kf16 = row_tops_kth(keys, rp.k, s) << 16;
   if (threadIdx.x == 0) s.n = 0;
   const float flmax = unord_f32((uint32_t)block_max_u64(ord_f32(pf.fl), s.red));  // (barriers)
   // the row floor (raw logits) and, per chunk, how much of its list can reach it
@@ -1084,21 +1068,19 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     // below every value), sorted: lane t holds the t-th largest.  The
     // kk-th largest gives the wave floor (its top 16 bits: the largest
     // prefix that kk lane maxima reach), lanes 0..kTopsPub-1 publish the
-    // largest lane maxima, lane kTops-1 the kTops-th (-inf fills)
+    // 2 kTopsPub largest lane maxima, lane kTops-1 the kTops-th (-inf fills)
     const uint32_t sk = wave_sort_desc(r.vok[0] ? radix_key(tv) : 0u);
     const bool some = kk <= (uint32_t)Lw;  // (kk - 1 is a lane: at most 63)
     wfloor = !kk ? 0xFFFFFFFFu : some ? ((uint32_t)__builtin_amdgcn_readlane((int)sk, (int)kk - 1) >> 16) << 16 : 0u;
     const float sv = sk > 0x007FFFFFu ? radix_value(sk) : -INFINITY;
-    float* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
-    if (lane < kTopsPub) tops[lane] = sv;
-    if (topk_more_tops(a.nchunks, rp.k)) {
-      if (lane >= kTopsPub && lane < 2 * kTopsPub) more_tops(a, b, c)[wave * kTopsPub + lane - kTopsPub] = sv;
-    }
+    uint32_t* tops = a.lane_tops + (((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub;
+    const uint32_t k16 = max(sk, 0x007FFFFFu) >> 16;
+    const uint32_t next = (uint32_t)__shfl((int)k16, (lane + kTopsPub) & 63, 64);
+    if (lane < kTopsPub) tops[lane] = k16 | (next << 16);
     if (lane == kTops - 1) sh.wtop[wave] = sv;
   } else if (topk && lane < kTopsPub) {
     if (lane == 0) sh.wtop[wave] = -INFINITY;
-    a.lane_tops[(((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub + lane] = -INFINITY;
-    if (topk_more_tops(a.nchunks, rp.k)) more_tops(a, b, c)[wave * kTopsPub + lane] = -INFINITY;
+    a.lane_tops[(((size_t)b * a.nchunks + c) * (kThreads / 64) + wave) * kTopsPub + lane] = 0x007F007Fu;  // -inf
   }
   if (lane == 0) { sh.wkey[wave] = wkey; sh.wfloor[wave] = wfloor; }
   if (threadIdx.x == 0) { sh.cnt = 0; sh.cnt_b = 0; sh.waves = 0; }
@@ -1212,14 +1194,13 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     slot_b = n_a + (uint32_t)__builtin_amdgcn_readfirstlane((int)wbase) + ((incl - mine) >> 16);
   }
   unsigned long long* out = a.cand + ((size_t)b * a.nchunks + c) * kCandCap;
-  const uint32_t cap = topk_more_tops(a.nchunks, rp.k) ? kCandCap - kMoreTops : kCandCap;  // entries of the list
   const bool restage = nst > (uint32_t)kScanStage;
 #pragma unroll
   for (int n = 0; n < kScanStage; ++n) {
     if (!restage && (uint32_t)n < nst) {  // the staged entries (the lane's own LDS column)
       const bool ta = (st_a >> n) & 1u;
       const uint32_t slot = ta ? slot_a : slot_b;
-      if (slot < cap) out[slot] = sh.stage[n][threadIdx.x];
+      if (slot < (uint32_t)kCandCap) out[slot] = sh.stage[n][threadIdx.x];
       slot_a += ta ? 1u : 0u;
       slot_b += ta ? 0u : 1u;
     }
@@ -1234,7 +1215,7 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
       if (l >= lo) {
         const bool ta = l >= th_a;
         const uint32_t slot = ta ? slot_a : slot_b;
-        if (slot < cap)
+        if (slot < (uint32_t)kCandCap)
           out[slot] = ((unsigned long long)radix_key(l / rp.tp) << 32) | (uint32_t)elem_index<VEC>(base, q * VEC + e);
         slot_a += ta ? 1u : 0u;
         slot_b += ta ? 0u : 1u;
@@ -1248,8 +1229,8 @@ __device__ __forceinline__ void scan_item(const SampleArgs& a, int b, int c, Chu
     if (done == kThreads / 64 - 1) {
       const uint32_t n_a = atomicAdd(&sh.cnt, 0u), n = n_a + atomicAdd(&sh.cnt_b, 0u);
       a.cand_floor[(size_t)b * a.nchunks + c] = theta_v;
-      a.cand_count[(size_t)b * a.nchunks + c] = n > cap ? kCandCap + 1 : n;
-      a.cand_count_a[(size_t)b * a.nchunks + c] = n_a > cap ? kCandCap + 1 : n_a;
+      a.cand_count[(size_t)b * a.nchunks + c] = n > (uint32_t)kCandCap ? kCandCap + 1 : n;
+      a.cand_count_a[(size_t)b * a.nchunks + c] = n_a;
       a.cand_floor_a[(size_t)b * a.nchunks + c] = th_a;
     }
   }
@@ -1499,7 +1480,6 @@ __global__ void __launch_bounds__(kThreads) topk_select_kernel(SampleArgs a, flo
   // the row's maximum key tells whether it holds a NaN
   unsigned long long mk = 0;
   for (int c = threadIdx.x; c < NC; c += blockDim.x) mk = max_u64(mk, a.chunk_max[(size_t)b * NC + c]);
-  topk_prefetch_more(a, b, K, pf);
   mk = block_max_u64(mk, s.red);
   bool fast = (uint32_t)(mk >> 32) != 0xFFFFFFFFu;
   if (fast) {
@@ -1828,7 +1808,6 @@ __global__ void __launch_bounds__(kThreads) sample_select_kernel(SampleArgs a) {
     return;
   }
   const bool fast_topk = rp.mode == ROW_FILTER && rp.k > 0 && rp.k <= kFastK;
-  if (fast_topk) topk_prefetch_more(a, b, rp.k, pf);
   const bool topp_only = rp.mode == ROW_FILTER && rp.k == 0 && rp.p < 1.0f;
   int tbm = INT_MIN;  // top-p-only rows: the chunks' top grid bins, loaded with the maxima
   if (topp_only)
@@ -2383,7 +2362,7 @@ static SampleArgs make_args(const void* logits, int dtype, int batch, int vocab,
   a.last_fill = ((vocab - (a.nchunks - 1) * a.chunk) * 8 + a.chunk - 1) / a.chunk;
 
   a.stride = row_stride;
-  a.lane_tops = (float*)(ws + w.lane_tops);
+  a.lane_tops = (uint32_t*)(ws + w.lane_tops);
   a.topp_chunk_hist = (uint32_t*)(ws + w.topp_chunk_hist);
   a.topp_chunk_tb = (int32_t*)(ws + w.topp_chunk_tb);
   a.row_ib = (int32_t*)(ws + w.row_ib);
