@@ -64,15 +64,16 @@ constexpr bool ring_takes_small(bool logits, int batch, int V, int cus) {
 // Whether it takes a sampled call of 65-128 rows: it costs about 21 + 33 t, 13 +
 // 40 t, 13 + 41 t or 16 + 49 t us for t tiles (a remainder of a few rows half a
 // tile) at 65-68, 69-80, 81-96 or more rows, the tile kernel's two passes 22 +
-// 0.17 r, 24 + 0.18 r, 28 + 0.16 r or 30 + 0.18 r for a share of r rows (V = 98,304 / 248,320, each call after a
-// pause, B = 80 92 / 183 us in the tile kernel against 92 / 162; B = 96 89 / 182
-// against 92 / 166; B = 128 101 / 197 against 109 / 194).
+// 0.17 r, 24 + 0.18 r, 28 + 0.16 r or 30 + 0.18 r for a share of r rows (V =
+// 40,960 / 98,304 / 248,320, each call after a pause: B = 80 56 / 92 / 183 us in the
+// tile kernel against 53 / 92 / 162; B = 96 56 / 89 / 182 against 54 / 92 / 166; B =
+// 128 63 / 101 / 197 against 63 / 109 / 194).
 constexpr bool ring_takes_sample(int batch, int V, int cus) {
   const int share = ring_share(V, cus), rem = share % 256;
   const int t8 = share / 256 * 8 + (rem == 0 ? 0 : rem <= 16 ? 4 : rem <= 32 ? 5 : 8);  // eighths of tiles
-  if (batch <= 68) return 8 * share >= 205 * t8;
-  if (batch <= 80) return 8 * share >= 225 * t8 - 480;
-  if (batch <= 96) return 8 * share >= 255 * t8 - 744;
+  if (batch <= 68) return 8 * share >= 230 * t8 - 600;
+  if (batch <= 80) return 8 * share >= 225 * t8 - 528;
+  if (batch <= 96) return 8 * share >= 255 * t8 - 768;
   return 8 * share >= 268 * t8 - 784;
 }
 
